@@ -157,6 +157,37 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// Maximum and sum over the four lanes (g, c), g = 0 .. 3, that hold one query
+// head's scores, on the row-swap moves of gfx950: v_permlane16_swap and
+// v_permlane32_swap of a register with itself leave both partners' values in
+// the lane. (An xor shuffle compiles to ds_bpermute with its address
+// arithmetic: two dependent LDS round trips in every step's softmax chain.)
+struct LanePair {
+  float x, y;
+};
+
+__device__ __forceinline__ LanePair pair_xor16(float v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+
+__device__ __forceinline__ LanePair pair_xor32(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+
+__device__ __forceinline__ float head_max(float v) {
+  const LanePair a = pair_xor16(v);
+  const LanePair b = pair_xor32(fmaxf(a.x, a.y));
+  return fmaxf(b.x, b.y);
+}
+
+__device__ __forceinline__ float head_sum(float v) {
+  const LanePair a = pair_xor16(v);
+  const LanePair b = pair_xor32(a.x + a.y);
+  return b.x + b.y;
+}
+
 // Orders this wave's LDS accesses in the compiler only. The LDS unit
 // executes one wave's DS instructions in issue order, so a write followed by
 // a read of the same bytes (by any lanes of the wave) needs no hardware wait;
@@ -836,8 +867,7 @@ struct MfmaDecoder {
           cmax = fmaxf(cmax, v);
         }
       }
-      cmax = fmaxf(cmax, __shfl_xor(cmax, 16, 64));
-      cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
+      cmax = head_max(cmax);
       const float mn = fmaxf(m[ht], cmax);  // finite: every chunk has a valid token
       const float alpha = __builtin_amdgcn_exp2f(m[ht] - mn);
       m[ht] = mn;
@@ -1010,10 +1040,7 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a) 
   // Per-lane partial denominators -> per head (sum over the 4 lane groups).
 #pragma unroll
   for (int ht = 0; ht < kHeadTiles; ++ht) {
-    float l = dec.lsum[ht];
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
-    dec.lsum[ht] = l;
+    dec.lsum[ht] = head_sum(dec.lsum[ht]);
   }
 
   const uint32_t heads = min(a.group, static_cast<uint32_t>(kHeadTiles * 16));
@@ -1571,15 +1598,13 @@ struct StreamDecoder {
     pv4 pb[kHT], pr[kHT];
 #pragma unroll
     for (int ht = 0; ht < kHT; ++ht) {
-      float cmax = -INFINITY;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float v = t0 + 4 * g + r < p1 ? s[ht][r] * sl2 : -INFINITY;
-        s[ht][r] = v;
-        cmax = fmaxf(cmax, v);
+      for (int r = 0; r < 4; ++r) s[ht][r] *= sl2;
+      if (t0 + kStep > p1) {  // uniform: only a partition's last step holds tokens past its end
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[ht][r] = t0 + 4 * g + r < p1 ? s[ht][r] : -INFINITY;
       }
-      cmax = fmaxf(cmax, __shfl_xor(cmax, 16, 64));
-      cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
+      const float cmax = head_max(fmaxf(fmaxf(s[ht][0], s[ht][1]), fmaxf(s[ht][2], s[ht][3])));
       const float mn = fmaxf(m[ht], cmax);  // finite: every step has a valid token
       // Rescale only when some head's maximum moved (exact; usually skipped).
       if (__builtin_amdgcn_ballot_w64(mn > m[ht]) != 0) {
@@ -2181,10 +2206,7 @@ __device__ __forceinline__ void stream_item(const DecodeArgs& a, uint8_t* tiles,
   float lt[kHT];
 #pragma unroll
   for (int ht = 0; ht < kHT; ++ht) {
-    float l = dec.lsum[ht];
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
-    lt[ht] = l;
+    lt[ht] = head_sum(dec.lsum[ht]);
   }
   if constexpr (kPair) {
     // Two partitions of one KV head per workgroup (pair_item): the odd one
@@ -2400,9 +2422,7 @@ __device__ __forceinline__ void stream_item_shared(const DecodeArgs& a, uint8_t*
 
 #pragma unroll
   for (int ht = 0; ht < kHTW; ++ht) {
-    float l = dec.lsum[ht];
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    const float l = head_sum(dec.lsum[ht]);
     if (h0 + ht * 16U + dec.c < a.group)
       store_wave_result<QE>(a, dec, ht, seq, kvh * a.group + h0 + ht * 16U, part, v_scale, l);
   }
