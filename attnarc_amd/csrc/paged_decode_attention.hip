@@ -24,8 +24,10 @@
 //   decode_mfma_kernel   the same head layout with 32-token chunks and K in
 //                        registers, for block sizes below 16 and partitions
 //                        that are not a multiple of 16 tokens.
-//   decode_vector_kernel any shape and dtype (including F32); fp32 VALU on
-//                        64-token tiles. Covers the general contract.
+//   (F32 queries and caches at head sizes 64-128 run the first two kernels
+//   on F32 MFMA: F32StreamDecoder.)
+//   decode_vector_kernel any shape and dtype; fp32 VALU on 64-token tiles.
+//                        Covers the general contract.
 //   merge_kernel / merge_rows_kernel / merge_wide_kernel
 //                        stable log-sum-exp merge of per-partition states
 //                        (the math of paged_decode_attention.cu:780-852).
@@ -1511,6 +1513,44 @@ struct StreamDecoder {
     }
   }
 
+  // f(dim, four consecutive dims of head 16 ht + c of the accumulated output).
+  template <typename F>
+  __device__ __forceinline__ void each_dims4(int ht, F&& f) const {
+#pragma unroll
+    for (int dt = 0; dt < kDt; ++dt) f(dt * 16U + 4U * g, acc[ht][dt]);
+  }
+
+  // Query heads head0 .. head0 + live - 1 of the item's sequence as MFMA B
+  // operands (absent heads and dims past the head size are zero). Waits for
+  // the step DMA issued before it as well: vmcnt counts both.
+  __device__ __forceinline__ void load_query(uint32_t seq, uint32_t head0, uint32_t live) {
+    u32x4 qw[kHT][kKc];
+    uint32_t dim[kKc];  // this lane's eight dims of chunk kc
+#pragma unroll
+    for (int kc = 0; kc < kKc; ++kc) dim[kc] = kFp8 ? ((kc >> 1) * 64 + g * 16 + ((kc ^ g) & 1U) * 8) : (kc * 32 + g * 8);
+#pragma unroll
+    for (int ht = 0; ht < kHT; ++ht) {
+      const uint32_t h = min(ht * 16U + c, live - 1U);  // rows past the group are zeroed below
+      const uint16_t* qrow =
+          static_cast<const uint16_t*>(a.query) + (static_cast<uint64_t>(seq) * a.query_heads + head0 + h) * kD;
+#pragma unroll
+      for (int kc = 0; kc < kKc; ++kc) vm_load16(qw[ht][kc], qrow + (dim[kc] < kD ? dim[kc] : 0U));
+    }
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+#pragma unroll
+    for (int ht = 0; ht < kHT; ++ht) {
+#pragma unroll
+      for (int kc = 0; kc < kKc; ++kc) asm volatile("" : "+v"(qw[ht][kc]));  // loaded: the wait above was vmcnt(0)
+    }
+#pragma unroll
+    for (int ht = 0; ht < kHT; ++ht) {
+      const bool in_group = ht * 16U + c < live;
+#pragma unroll
+      for (int kc = 0; kc < kKc; ++kc)
+        qb[ht][kc] = __builtin_bit_cast(vec8, in_group && dim[kc] < kD ? qw[ht][kc] : u32x4{0U, 0U, 0U, 0U});
+    }
+  }
+
   __device__ __forceinline__ void qk(const uint8_t* stage, f32x4 (&z)[kHT]) const {
     vec8 kop[kKc];
 #pragma unroll
@@ -1649,6 +1689,218 @@ struct StreamDecoder {
     }
   }
 };
+
+// F32 queries over F32 caches on the streaming kernels, groups of up to 16
+// heads: the interface of StreamDecoder on v_mfma_f32_16x16x4_f32 (products
+// and sums in F32). Bound by HBM: a 16-token step of one KV head is 128 kD
+// bytes against kD / 2 MFMAs of 32 cycles, a third of the time those bytes
+// take a CU at head size 128. Measured against the 64-token VALU tiles of
+// decode_vector_kernel, whose waves wait for each tile's loads (call us): 16
+// sequences x 255-4093 tokens, Hq 32 / Hkv 8, head size 128 115 -> 57 (2.5 ->
+// 5.0 TB/s), 80 98 -> 43, 64 71 -> 37; 48 x <= 2000 tokens at 128 176 -> 86.
+//   S: lane (g, c) reads K row c's 16-byte chunk 4 kc + g (dims 16 kc + 4g ..
+//      + 3) and Q head c's same dims; MFMA j takes element j of both, so a
+//      chunk is one LDS read and four MFMAs, and S[token 4g + r][head c] lands
+//      in lane (g, c), which is PV's B operand for K index g of MFMA r.
+//   O: MFMA r's A operand is V row 4g + r. A lane reads four consecutive dims
+//      64 b + 4c .. + 3 and uses element j as the A operand of tile (b, j), so
+//      tile (b, j)'s row i is dim 64 b + 4i + j. Dims past the last whole 64
+//      (head sizes 80, 96, 112) come as tiles of two (32 b + 2i + j) and one
+//      (16 b + i) elements per lane.
+template <uint32_t kD, int kS = kStreamStages, int kNt = -1>
+struct F32StreamDecoder {
+  static_assert(kD % 16 == 0 && kD >= 64 && kD <= 128, "whole 16-dim tiles");
+  static constexpr bool kNtKV = kNt >= 0 ? kNt != 0 : (kD * 4U) % 128U == 0;
+  static constexpr int kHT = 1;
+  static constexpr int kDt = kD / 16;                 // accumulator tiles
+  static constexpr int kKc = kD / 16;                 // 16-dim QK chunks of a lane group
+  static constexpr uint32_t kPitch = kD * 4;          // bytes of a row
+  static constexpr uint32_t kRowChunks = kD / 4;      // 16-byte chunks of a row
+  static constexpr bool kEvenRows = 64U % kRowChunks == 0;  // a DMA instruction brings whole rows
+  static constexpr uint32_t kRowsPerDma = kEvenRows ? 64U / kRowChunks : 0U;
+  static constexpr int kDma = kD / 16;                // 1 KiB DMA instructions per tensor per step
+  static constexpr int kStages = kS;
+  static constexpr uint32_t kVOff = kStep * kPitch;
+  static constexpr uint32_t kStageBytes = 2 * kVOff;
+  static constexpr uint32_t kVTileOff = 0;            // PV reads V in place
+  static constexpr uint32_t kWaveBytes = kStages * kStageBytes;
+  static constexpr int kDmaPerStep = 2 * kDma;
+  static constexpr uint32_t kElem = 4;
+  // K row r keeps chunk L at (L + (r >> kRotShift)) mod kRowChunks: the 16
+  // rows of one operand read then cover all banks (row pitches repeat over the
+  // 256 bytes of banks after 1, 2 or 4 rows). V rows are read along the row.
+  static constexpr uint32_t kRotShift = kPitch % 256U == 0 ? 0U : kPitch % 128U == 0 ? 1U : 2U;
+
+  const DecodeArgs& a;
+  uint32_t lane, g, c;
+  uint32_t p1;
+  uint32_t len;
+  uint32_t last_block;
+  const int32_t* table;
+  uint64_t kbase, vbase;
+  uint64_t kstride_b, vstride_b, kstride_p, vstride_p;
+  uint32_t k_voff[kDma], v_voff[kEvenRows ? 1 : kDma];  // lane's DMA offsets
+  uint32_t k_off[kKc];                                  // lane's operand offsets in a K tile
+  float sl2;
+
+  f32x4 q[kKc];
+  f32x4 acc[1][kDt];
+  float m[1];
+  float lsum[1];
+
+  __device__ __forceinline__ F32StreamDecoder(const DecodeArgs& args) : a(args) {}
+
+  __device__ __forceinline__ uint32_t block_of(uint32_t t0) const {
+    const uint32_t lb = min(t0 >> a.block_shift, last_block);
+    using ConstWord = const __attribute__((address_space(4))) int32_t;
+    return static_cast<uint32_t>(((ConstWord*)table)[lb]);
+  }
+
+  __device__ __forceinline__ uint64_t row_base(uint64_t base, uint64_t stride_b, uint64_t stride_p, uint32_t blk,
+                                               uint32_t t0) const {
+    return base + blk * stride_b + (t0 & (a.block_size - 1U)) * stride_p;
+  }
+
+  __device__ __forceinline__ void init_offsets() {
+#pragma unroll
+    for (int i = 0; i < kDma; ++i) {
+      const uint32_t idx = 64U * i + lane;
+      const uint32_t r = idx / kRowChunks, slot = idx % kRowChunks;
+      const uint32_t chunk = (slot + kRowChunks - (r >> kRotShift) % kRowChunks) % kRowChunks;
+      // with whole rows per instruction the row part beyond the first is scalar (issue)
+      k_voff[i] = static_cast<uint32_t>((kEvenRows ? r - i * kRowsPerDma : r) * kstride_p) + (chunk << 4);
+      if (!kEvenRows || i == 0) v_voff[i] = static_cast<uint32_t>(r * vstride_p) + (slot << 4);
+    }
+#pragma unroll
+    for (int kc = 0; kc < kKc; ++kc)
+      k_off[kc] = c * kPitch + ((4U * kc + g + (c >> kRotShift)) % kRowChunks) * 16U;
+  }
+
+  __device__ __forceinline__ void issue(uint8_t* stage, uint32_t blk, uint32_t t0) const {
+    const uint64_t kb = row_base(kbase, kstride_b, kstride_p, blk, t0);
+    const uint64_t vb = row_base(vbase, vstride_b, vstride_p, blk, t0);
+#pragma unroll
+    for (int i = 0; i < kDma; ++i)
+      vm_load16_lds_sv<kNtKV>(k_voff[i], kb + i * kRowsPerDma * kstride_p, stage + i * 1024);
+#pragma unroll
+    for (int i = 0; i < kDma; ++i)
+      vm_load16_lds_sv<kNtKV>(v_voff[kEvenRows ? 0 : i], vb + i * kRowsPerDma * vstride_p, stage + kVOff + i * 1024);
+  }
+
+  __device__ __forceinline__ void load_query(uint32_t seq, uint32_t head0, uint32_t live) {
+    const uint32_t h = min(c, live - 1U);  // rows past the group are zeroed below
+    const float* qrow = static_cast<const float*>(a.query) + (static_cast<uint64_t>(seq) * a.query_heads + head0 + h) * kD;
+#pragma unroll
+    for (int kc = 0; kc < kKc; ++kc) q[kc] = *reinterpret_cast<const f32x4*>(qrow + 16 * kc + 4 * g);
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+#pragma unroll
+    for (int kc = 0; kc < kKc; ++kc) q[kc] = c < live ? q[kc] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+
+  __device__ __forceinline__ void qk(const uint8_t* stage, f32x4 (&z)[1]) const {
+    f32x4 z0 = {0.0f, 0.0f, 0.0f, 0.0f}, z1 = z0;  // two chains: half the dependent MFMAs and roundings each
+#pragma unroll
+    for (int kc = 0; kc < kKc; ++kc) {
+      const f32x4 k = *reinterpret_cast<const f32x4*>(stage + k_off[kc]);
+      z0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[0], q[kc][0], z0, 0, 0, 0);
+      z1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[1], q[kc][1], z1, 0, 0, 0);
+      z0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[2], q[kc][2], z0, 0, 0, 0);
+      z1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[3], q[kc][3], z1, 0, 0, 0);
+    }
+    z[0] = z0 + z1;
+  }
+
+  // Rows of tokens past the sequence end (possible only in its last step):
+  // zeroed so that P = 0 meets a finite V. A quarter wave per row.
+  __device__ __forceinline__ void zero_dead_rows(uint8_t* tile, uint32_t t0) const {
+    if (t0 + kStep <= len) return;  // uniform
+#pragma unroll
+    for (uint32_t r = 0; r < 4; ++r) {
+      if (t0 + 4 * g + r >= len) {
+#pragma unroll
+        for (uint32_t ch = 0; ch < (kRowChunks + 15) / 16; ++ch) {
+          if (ch * 16 + c < kRowChunks)
+            *reinterpret_cast<u32x4*>(tile + (4 * g + r) * kPitch + (ch * 16 + c) * 16) = u32x4{0U, 0U, 0U, 0U};
+        }
+      }
+    }
+  }
+
+  // PV tiles of kE elements per lane from dim kBase on: tile (j) row i is dim
+  // kBase + kE i + j.
+  template <uint32_t kBase, uint32_t kE>
+  __device__ __forceinline__ void pv_tiles(const uint8_t* tile, const f32x4& p) {
+    typedef float vec __attribute__((ext_vector_type(kE)));
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float e[kE];
+      if constexpr (kE == 1) {
+        e[0] = *reinterpret_cast<const float*>(tile + (4 * g + r) * kPitch + (kBase + c) * 4);
+      } else {
+        const vec v = *reinterpret_cast<const vec*>(tile + (4 * g + r) * kPitch + (kBase + kE * c) * 4);
+#pragma unroll
+        for (uint32_t j = 0; j < kE; ++j) e[j] = v[j];
+      }
+#pragma unroll
+      for (uint32_t j = 0; j < kE; ++j)
+        acc[0][kBase / 16 + j] = __builtin_amdgcn_mfma_f32_16x16x4f32(e[j], p[r], acc[0][kBase / 16 + j], 0, 0, 0);
+    }
+  }
+
+  __device__ __forceinline__ void softmax_pv(f32x4 (&s)[1], uint32_t t0, const uint8_t* tile) {
+    f32x4 x = s[0] * sl2;
+    if (t0 + kStep > p1) {  // uniform
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x[r] = t0 + 4 * g + r < p1 ? x[r] : -INFINITY;
+    }
+    const float mn = fmaxf(m[0], head_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]))));
+    if (__builtin_amdgcn_ballot_w64(mn > m[0]) != 0) {
+      const float alpha = __builtin_amdgcn_exp2f(m[0] - mn);
+      lsum[0] *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < kDt; ++dt) acc[0][dt] *= alpha;
+      m[0] = mn;
+    }
+    f32x4 p;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(x[r] - m[0]);
+    lsum[0] += (p[0] + p[1]) + (p[2] + p[3]);
+    pv_tiles<0, 4>(tile, p);
+    if constexpr (kD == 128) pv_tiles<64, 4>(tile, p);
+    if constexpr (kD % 64 >= 32) pv_tiles<kD / 64 * 64, 2>(tile, p);
+    if constexpr (kD % 32 == 16) pv_tiles<kD / 32 * 32, 1>(tile, p);
+  }
+
+  // f(dim, four consecutive dims of head c of the accumulated output).
+  template <typename F>
+  __device__ __forceinline__ void each_dims4(int, F&& f) const {
+    constexpr int kFull = kD / 64 * 4;
+#pragma unroll
+    for (int b = 0; b < kFull; b += 4) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        f(16U * b + 16U * g + 4U * r, f32x4{acc[0][b][r], acc[0][b + 1][r], acc[0][b + 2][r], acc[0][b + 3][r]});
+    }
+    if constexpr (kD % 64 >= 32) {
+#pragma unroll
+      for (int r = 0; r < 4; r += 2)
+        f(16U * kFull + 8U * g + 2U * r,
+          f32x4{acc[0][kFull][r], acc[0][kFull + 1][r], acc[0][kFull][r + 1], acc[0][kFull + 1][r + 1]});
+    }
+    if constexpr (kD % 32 == 16) f(16U * (kDt - 1) + 4U * g, acc[0][kDt - 1]);
+  }
+};
+
+template <typename QE, bool kFp8, int kHT, uint32_t kD, int kS, int kNt>
+struct DecoderOf {
+  using type = StreamDecoder<QE, kFp8, kHT, kD, kS, kNt>;
+};
+template <uint32_t kD, int kS, int kNt>
+struct DecoderOf<F32Elem, false, 1, kD, kS, kNt> {
+  using type = F32StreamDecoder<kD, kS, kNt>;
+};
+template <typename QE, bool kFp8, int kHT, uint32_t kD, int kS, int kNt>
+using Decoder = typename DecoderOf<QE, kFp8, kHT, kD, kS, kNt>::type;
 
 // Per-wave timeline of the streaming kernels, compiled only into profiling
 // builds (-DLOOM_HIP_WAVE_TRACE, attnarc_amd/wave_trace.py): each wave of an
@@ -1894,21 +2146,24 @@ template <typename QE, bool kNt = false, typename Dec>
 __device__ __forceinline__ void store_wave_result(const DecodeArgs& a, const Dec& dec, int ht, uint32_t seq,
                                                   uint32_t head0, uint32_t part, float v_scale, float l) {
   constexpr uint32_t D = Dec::kDt * 16;
+  using QT = typename QE::T;
   const uint64_t row = static_cast<uint64_t>(seq) * a.query_heads + head0 + dec.c;
   if (a.parts == 1) {
     const float inv = v_scale / l;
-    uint16_t* o = static_cast<uint16_t*>(a.output) + row * D + 4 * dec.g;
-#pragma unroll
-    for (int dt = 0; dt < Dec::kDt; ++dt) {
-      uint32_t w0 = QE::from_f(dec.acc[ht][dt][0] * inv) | (static_cast<uint32_t>(QE::from_f(dec.acc[ht][dt][1] * inv)) << 16);
-      uint32_t w1 = QE::from_f(dec.acc[ht][dt][2] * inv) | (static_cast<uint32_t>(QE::from_f(dec.acc[ht][dt][3] * inv)) << 16);
-      *reinterpret_cast<uint2*>(o + dt * 16) = make_uint2(w0, w1);
-    }
+    QT* out = static_cast<QT*>(a.output) + row * D;
+    dec.each_dims4(ht, [&](uint32_t dim, f32x4 o) {
+      if constexpr (sizeof(QT) == 4) {
+        *reinterpret_cast<f32x4*>(out + dim) = o / l;
+      } else {
+        const uint32_t w0 = QE::from_f(o[0] * inv) | (static_cast<uint32_t>(QE::from_f(o[1] * inv)) << 16);
+        const uint32_t w1 = QE::from_f(o[2] * inv) | (static_cast<uint32_t>(QE::from_f(o[3] * inv)) << 16);
+        *reinterpret_cast<uint2*>(out + dim) = make_uint2(w0, w1);
+      }
+    });
     if (a.lse != nullptr && dec.g == 0) a.lse[row] = (dec.m[ht] + log2f(l)) * kLn2;
   } else {
     const uint64_t state = state_of(a, row, part);
-#pragma unroll
-    for (int dt = 0; dt < Dec::kDt; ++dt) put_partial4<kNt>(a, state * D + 4 * dec.g + dt * 16, dec.acc[ht][dt], v_scale);
+    dec.each_dims4(ht, [&](uint32_t dim, f32x4 o) { put_partial4<kNt>(a, state * D + dim, o, v_scale); });
     if (dec.g == 0) {
       a.ws_ml[state * 2] = dec.m[ht];
       a.ws_ml[state * 2 + 1] = l;
@@ -2058,8 +2313,7 @@ __device__ __forceinline__ void stream_item(const DecodeArgs& a, uint8_t* tiles,
                                             bool preloaded = false, const uint32_t* first_blocks = nullptr,
                                             uint8_t* partner = nullptr) {
   static_assert(kHT == 1 || kSplit == 1, "two head tiles run one wave per item");
-  using Dec = StreamDecoder<QE, kFp8, kHT, kD, kS, kNt>;
-  using vec8 = typename Dec::vec8;
+  using Dec = Decoder<QE, kFp8, kHT, kD, kS, kNt>;
   constexpr int S = Dec::kStages;
   const uint32_t kvh = item.kvh;
   const uint32_t part = item.part;
@@ -2140,36 +2394,7 @@ __device__ __forceinline__ void stream_item(const DecodeArgs& a, uint8_t* tiles,
     }
     // Q is loaded after the first steps' K/V and waited for together with
     // them, so a wave's start costs one memory round trip, not two.
-    {
-      u32x4 qw[kHT][Dec::kKc];
-#pragma unroll
-      for (int ht = 0; ht < kHT; ++ht) {
-        const uint32_t h = min(ht * 16U + dec.c, a.group - 1U);  // rows >= group are zeroed below
-        const uint16_t* qrow = static_cast<const uint16_t*>(a.query) +
-                               (static_cast<uint64_t>(seq) * a.query_heads + kvh * a.group + h) * kD;
-#pragma unroll
-        for (int kc = 0; kc < Dec::kKc; ++kc) {
-          const uint32_t dim = kFp8 ? ((kc >> 1) * 64 + dec.g * 16 + ((kc ^ dec.g) & 1U) * 8) : (kc * 32 + dec.g * 8);
-          vm_load16(qw[ht][kc], qrow + (dim < kD ? dim : 0U));  // dims past the head size are zeroed below
-        }
-      }
-      asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-#pragma unroll
-      for (int ht = 0; ht < kHT; ++ht) {
-#pragma unroll
-        for (int kc = 0; kc < Dec::kKc; ++kc) asm volatile("" : "+v"(qw[ht][kc]));  // loaded: the wait above was vmcnt(0)
-      }
-#pragma unroll
-      for (int ht = 0; ht < kHT; ++ht) {
-        const bool live = ht * 16U + dec.c < a.group;
-#pragma unroll
-        for (int kc = 0; kc < Dec::kKc; ++kc) {
-          const uint32_t dim = kFp8 ? ((kc >> 1) * 64 + dec.g * 16 + ((kc ^ dec.g) & 1U) * 8) : (kc * 32 + dec.g * 8);
-          const bool in_row = dim < kD;
-          dec.qb[ht][kc] = __builtin_bit_cast(vec8, live && in_row ? qw[ht][kc] : u32x4{0U, 0U, 0U, 0U});
-        }
-      }
-    }
+    dec.load_query(seq, kvh * a.group, a.group);
     LOOM_WAVE_STALL_DECL;
     for (uint32_t n = 0; n < my_n; n += S) {
       LOOM_WAVE_MARK(n, S, my_n);
@@ -2181,7 +2406,7 @@ __device__ __forceinline__ void stream_item(const DecodeArgs& a, uint8_t* tiles,
           // this step's loads; the later steps' (up to S - 1) stay in flight
           LOOM_WAVE_STALL(n + i, my_n, (vm_wait_dma_later<Dec::kDmaPerStep, S - 1>(my_n - 1 - (n + i))));
           scalar_ready(nx[i]);
-          if (kFp8) {
+          if constexpr (kFp8) {
             dec.stage_v_fp8(tl[i], vtile, t0);
           } else {
             dec.zero_dead_rows(vtile, t0);
@@ -2246,8 +2471,7 @@ __device__ __forceinline__ void stream_item(const DecodeArgs& a, uint8_t* tiles,
     red_ml[wave][h][0] = dec.m[0];
     red_ml[wave][h][1] = l;
   }
-#pragma unroll
-  for (int dt = 0; dt < Dec::kDt; ++dt) *reinterpret_cast<f32x4*>(&red_o[wave][h][dt * 16 + 4 * dec.g]) = dec.acc[0][dt];
+  dec.each_dims4(0, [&](uint32_t dim, f32x4 o) { *reinterpret_cast<f32x4*>(&red_o[wave][h][dim]) = o; });
   __syncthreads();
   const uint32_t heads = min(a.group, 16U);
   for (uint32_t idx = threadIdx.x; idx < heads * kD; idx += kSplit * 64) {
@@ -2265,7 +2489,7 @@ __device__ __forceinline__ void stream_item(const DecodeArgs& a, uint8_t* tiles,
     O *= v_scale;
     const uint64_t row = static_cast<uint64_t>(seq) * a.query_heads + kvh * a.group + hl;
     if (a.parts == 1) {
-      static_cast<uint16_t*>(a.output)[row * kD + d] = QE::from_f(O / L);
+      static_cast<typename QE::T*>(a.output)[row * kD + d] = QE::from_f(O / L);
       if (a.lse != nullptr && d == 0) a.lse[row] = (M + log2f(L)) * kLn2;
     } else {
       const uint64_t state = state_of(a, row, part);
@@ -2297,7 +2521,6 @@ constexpr int kSharedStages = 4;
 template <typename QE, bool kFp8, int kWaves, uint32_t kD, int kHTW = 2>
 __device__ __forceinline__ void stream_item_shared(const DecodeArgs& a, uint8_t* tiles, const WorkItem& item) {
   using Dec = StreamDecoder<QE, kFp8, kHTW, kD>;
-  using vec8 = typename Dec::vec8;
   constexpr int S = kSharedStages;
   const uint32_t kvh = item.kvh, part = item.part, seq = item.seq, len = item.len;
   const uint32_t p0 = part * a.partition_tokens;
@@ -2356,33 +2579,7 @@ __device__ __forceinline__ void stream_item_shared(const DecodeArgs& a, uint8_t*
       if (i < nst) dec.issue(tiles + i * Dec::kStageBytes, bk[i], p0 + i * kStep);
     }
   }
-  {
-    u32x4 qw[kHTW][Dec::kKc];
-#pragma unroll
-    for (int ht = 0; ht < kHTW; ++ht) {
-      const uint32_t h = min(h0 + ht * 16U + dec.c, a.group - 1U);  // rows >= group are zeroed below
-      const uint16_t* qrow = static_cast<const uint16_t*>(a.query) +
-                             (static_cast<uint64_t>(seq) * a.query_heads + kvh * a.group + h) * kD;
-#pragma unroll
-      for (int kc = 0; kc < Dec::kKc; ++kc) {
-        const uint32_t dim = kFp8 ? ((kc >> 1) * 64 + dec.g * 16 + ((kc ^ dec.g) & 1U) * 8) : (kc * 32 + dec.g * 8);
-        vm_load16(qw[ht][kc], qrow + dim);
-      }
-    }
-    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-#pragma unroll
-    for (int ht = 0; ht < kHTW; ++ht) {
-#pragma unroll
-      for (int kc = 0; kc < Dec::kKc; ++kc) asm volatile("" : "+v"(qw[ht][kc]));  // loaded: the wait above was vmcnt(0)
-    }
-#pragma unroll
-    for (int ht = 0; ht < kHTW; ++ht) {
-      const bool live = h0 + ht * 16U + dec.c < a.group;
-#pragma unroll
-      for (int kc = 0; kc < Dec::kKc; ++kc)
-        dec.qb[ht][kc] = __builtin_bit_cast(vec8, live ? qw[ht][kc] : u32x4{0U, 0U, 0U, 0U});
-    }
-  }
+  dec.load_query(seq, kvh * a.group + h0, a.group - h0);
 
   LOOM_WAVE_STALL_DECL;
   for (uint32_t n = 0; n < nst; n += S) {
@@ -2468,7 +2665,7 @@ template <typename QE, bool kFp8, int kSplit, int kHT = 1, uint32_t kD = kDim, i
 __global__ __launch_bounds__(kSplit * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void decode_stream_kernel(DecodeArgs a) {
   constexpr int kS = kFp8 ? kStreamStagesFp8 : kStreamStages;
-  using Dec = StreamDecoder<QE, kFp8, kHT, kD, kS, kNt>;
+  using Dec = Decoder<QE, kFp8, kHT, kD, kS, kNt>;
   __shared__ __attribute__((aligned(16))) uint8_t tiles[kSplit * Dec::kWaveBytes];
   LOOM_WAVE_STAMP(blockIdx.x * kSplit + (threadIdx.x >> 6));
   const WorkItem item = schedule_item(a, blockIdx.x);
@@ -2542,7 +2739,7 @@ template <typename QE, bool kFp8, int kGroup, uint32_t kD = kDim, int kNt = -1, 
 __global__ __launch_bounds__(kGroup * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void decode_stream_group_kernel(DecodeArgs a) {
   constexpr int kGroupStages = kFp8 ? kStreamStagesFp8 : kStreamGroupStages;
-  using Dec = StreamDecoder<QE, kFp8, 1, kD, kGroupStages, kNt>;
+  using Dec = Decoder<QE, kFp8, 1, kD, kGroupStages, kNt>;
   __shared__ __attribute__((aligned(16))) uint8_t tiles[kGroup * Dec::kWaveBytes];
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   LOOM_WAVE_STAMP(blockIdx.x * kGroup + wave);
@@ -3215,7 +3412,7 @@ bool stream_eligible(const Problem& p, uint64_t parts, uint32_t group) {
   if (parts > 1 && p.partition_tokens % kStep != 0) return false;
   const uint64_t es = cache_elem_size(p);
   const uint64_t limit = 1ULL << 31;
-  return 15 * p.k_page * es + 256 < limit && 15 * p.v_page * es + 256 < limit;
+  return 15 * p.k_page * es + 1024 < limit && 15 * p.v_page * es + 1024 < limit;
 }
 
 // Head size 64 on the streaming kernel: 16-bit queries, native or FP8 cache,
@@ -3343,6 +3540,63 @@ bool narrow_stream_eligible(const Problem& p, uint64_t parts, uint32_t group) {
 }
 
 
+// F32 queries over F32 caches on the streaming kernels: head sizes 64-128 of
+// the 16-bit path, at most 16 query heads per KV head (one head tile), blocks of a
+// power of two >= 16 tokens, partitions of whole steps, 16-byte aligned rows
+// and 31-bit lane offsets. Everything else stays on decode_vector_kernel;
+// head size 256 does because a wave's stages would take 64 KiB (16 x <= 4093
+// tokens, Hq 32 / Hkv 8: 205 us there, 224 here; 4 x <= 256 tokens 17.8
+// against 32.2).
+bool f32_stream_eligible(const Problem& p, uint64_t parts, uint32_t group) {
+  if (p.dtype != kF32 || p.cache_encoding != LOOM_HIP_KV_CACHE_NATIVE || p.value_head_size != p.head_size || group > 16)
+    return false;
+  const uint32_t d = p.head_size;
+  if (d != 64 && d != 80 && d != 96 && d != 112 && d != 128) return false;
+  if (!is_pow2(p.block_size) || !stream_eligible(p, parts, group)) return false;
+  const uint64_t strides[] = {p.k_block, p.k_page, p.k_head, p.v_block, p.v_page, p.v_head};
+  for (uint64_t st : strides) {
+    if (st % 4 != 0) return false;
+  }
+  // outputs and partial states are stored as 16-byte vectors
+  const bool stores = parts > 1 ? aligned16(p.workspace + static_cast<uint64_t>(p.sequences) * p.query_heads * parts * 2)
+                                : aligned16(p.output);
+  return aligned16(p.query) && aligned16(p.key_cache) && aligned16(p.value_cache) && stores;
+}
+
+// A wave's stages take 256 kD bytes of LDS, so the waves that a CU holds
+// decide the launch shape. Head size 64 (16 KiB, as 16-bit rows at 128) takes
+// that path's shapes. Larger heads: a 4-wave split fills a CU alone, so it runs
+// up to one workgroup per CU, two waves per item up to 1024 items and one wave
+// per item above; from 2048 items the pairing of adjacent heads outweighs the
+// coarser workgroups. Call us at head size 128 with 4 / 2 / 1 waves per item and
+// grouped: 256 items x <= 300 tokens 18.4 / 23.2 / 32.3 / 38.0, 512 x <= 512
+// 44.9 / 36.1 / 53.1 / 60.9, 1024 x <= 512 73.5 / 77.4 / 57.3 / 64.6, 3072 x
+// <= 256 120 / 96.2 / 88.8 / 85.1.
+template <uint32_t kD, int kNt>
+int launch_f32_stream_nt(const DecodeArgs& args, uint64_t grid, uint32_t steps, hipStream_t stream) {
+  constexpr bool kSmall = kD == 64;
+  if (grid >= 4096 || (grid >= (kSmall ? 1024 : 2048) && steps >= 8))
+    return launch_stream_group<F32Elem, false, kD, kD <= 80 ? 4 : 2, kNt>(args, grid, stream);
+  if (steps < 8 || grid >= 1024) return launch_stream<F32Elem, false, 1, 1, kD, kNt>(args, grid, stream);
+  if (!kSmall && grid > 256) return launch_stream<F32Elem, false, 2, 1, kD, kNt>(args, grid, stream);
+  return launch_stream<F32Elem, false, 4, 1, kD, kNt>(args, grid, stream);
+}
+
+int launch_f32_stream(const DecodeArgs& args, uint64_t grid, uint32_t steps, hipStream_t stream) {
+  // Rows of 320 and 448 bytes share 128-byte lines: the non-temporal hint
+  // only where each KV head's token rows are contiguous (HND).
+  const bool dense = args.k_page == args.head_size && args.v_page == args.head_size;
+  switch (args.head_size) {
+    case 64: return launch_f32_stream_nt<64, -1>(args, grid, steps, stream);
+    case 80: return dense ? launch_f32_stream_nt<80, 1>(args, grid, steps, stream)
+                          : launch_f32_stream_nt<80, -1>(args, grid, steps, stream);
+    case 96: return launch_f32_stream_nt<96, -1>(args, grid, steps, stream);
+    case 112: return dense ? launch_f32_stream_nt<112, 1>(args, grid, steps, stream)
+                           : launch_f32_stream_nt<112, -1>(args, grid, steps, stream);
+    default: return launch_f32_stream_nt<128, -1>(args, grid, steps, stream);
+  }
+}
+
 template <typename QE, typename CE, bool kVecK, uint32_t kDvl, bool kQLds, uint32_t kH>
 int launch_vector_kernel(const DecodeArgs& args, uint64_t grid, hipStream_t stream) {
   g_launch_kernel = "decode_vector_kernel";
@@ -3441,13 +3695,21 @@ int run_typed(const Problem& p, hipStream_t stream) {
   g_launch_pairs = false;
 
   int status = LOOM_HIP_SUCCESS;
-  bool use_narrow = false, use_mfma = false, use_heads = false;
-  if constexpr (!std::is_same<QE, F32Elem>::value) {
+  bool use_narrow = false, use_mfma = false, use_heads = false, use_f32 = false;
+  if constexpr (std::is_same<QE, F32Elem>::value) {
+    use_f32 = f32_stream_eligible(p, parts, group);
+  } else {
     use_heads = heads_stream_eligible(p, parts);
     use_narrow = !use_heads && narrow_stream_eligible(p, parts, group);
     use_mfma = !use_heads && !use_narrow && mfma_eligible(p);
   }
-  if (use_heads) {
+  if (use_f32) {
+    const uint64_t grid = parts * p.kv_heads * static_cast<uint64_t>(p.sequences);
+    if (grid > static_cast<uint64_t>(std::numeric_limits<int>::max()))
+      return fail(LOOM_HIP_UNSUPPORTED, "paged decode grid exceeds the launch limit");
+    args.grid_y = p.kv_heads;
+    status = launch_f32_stream(args, grid, (partition_tokens + kStep - 1) / kStep, stream);
+  } else if (use_heads) {
     if constexpr (!std::is_same<QE, F32Elem>::value) {
       const uint64_t grid = parts * p.kv_heads * static_cast<uint64_t>(p.sequences);
       if (grid > static_cast<uint64_t>(std::numeric_limits<int>::max()))

@@ -276,7 +276,8 @@ int loom_hip_paged_decode_attention_extended_no_alloc(
  * >= 16), "mfma" for the 32-token matrix-core kernel or "vector" for the
  * general kernel. A call whose partition size is not a multiple of 16 moves
  * from "mfma-stream" to "mfma"; one whose strides or pointers are not 16-byte
- * aligned moves to "vector".
+ * aligned moves to "vector". F32 queries report "vector" whichever kernel runs
+ * (loom_hip_last_kernel_name tells it).
  */
 int loom_hip_paged_decode_attention_supports(
     uint32_t dtype, uint32_t cache_encoding, uint32_t sequences,
