@@ -1220,23 +1220,31 @@ __device__ __forceinline__ void vm_load16_lds_sv(uint32_t voff, uint64_t base, u
 
 __device__ __forceinline__ void scalar_ready(uint32_t& v) { asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(v)); }
 
-// Pipeline stages per wave: a 16-bit stage is 8 KiB of K/V rows, an FP8
-// stage 4 KiB. Deeper pipelines measured no faster (FP8 with 2, 3 and 4
-// stages ran C4 at the same speed; two head tiles per wave ran C5 slower
-// with 4 and 6 stages than with 2).
+// Physical blocks of one step's tokens, 16 tokens each.
+template <int kN>
+struct StepBlocks {
+  uint32_t id[kN];
+  __device__ __forceinline__ void ready() {
+#pragma unroll
+    for (int i = 0; i < kN; ++i) scalar_ready(id[i]);
+  }
+};
+
+// Pipeline stages per wave: a 16-bit stage is 16 tokens (8 KiB of K/V rows at
+// head size 128), an FP8 stage 32 tokens (the same bytes). Deeper pipelines
+// measured no faster (two head tiles per wave ran C5 slower with 4 and 6
+// stages than with 2).
 constexpr int kStreamStages = 2;
-constexpr int kStreamStagesFp8 = 2;
 
 // kHT: 16-query-head tiles per wave (1, or 2 for groups of 17-32 heads). The
 // tiles share each step's K operand fetches and V transposed reads.
-// kD: head size (= value head size): 128; 64, where 16-bit rows of 128 bytes
-// take the FP8 path's DMA geometry (eight rows per instruction) without a
-// conversion and FP8 rows of 64 bytes come sixteen per instruction; or 256
-// with one head tile (16-bit rows of 512 bytes two per instruction, FP8 rows
-// of 256 bytes four per instruction).
-template <typename QE, bool kFp8, int kHT = 1, uint32_t kD = kDim,
-          int kS = kFp8 ? kStreamStagesFp8 : kStreamStages, int kNt = -1>
+// kD: head size (= value head size): 128; 64, whose rows of 128 bytes come
+// eight per DMA instruction; or 256 with one head tile (rows of 512 bytes, two
+// per instruction). 16-bit caches; FP8 ones take Fp8StreamDecoder.
+template <typename QE, int kHTiles = 1, uint32_t kD = kDim, int kS = kStreamStages, int kNt = -1>
 struct StreamDecoder {
+  static constexpr int kHT = kHTiles;
+  static constexpr uint32_t kTok = kStep;  // tokens per step
   static_assert(kD == kDim || kD == 64 || ((kD == 80 || kD == 96 || kD == 112 || kD == 256) && kHT == 1),
                 "head size 64, 128, or 80 / 96 / 112 / 256 with one head tile");
   // K/V loads carry the non-temporal hint when a cache row is whole 128-byte
@@ -1250,11 +1258,9 @@ struct StreamDecoder {
   // rows are contiguous (HND), so a step of 16 rows covers whole lines at
   // any head size (HND, 8-10% faster with it: 16-bit D80 178 -> 162 us, D96
   // 176 -> 161, D112 165 -> 152, FP8 D64 104 -> 95, D96 119 -> 115).
-  static constexpr bool kNtKV = kNt >= 0 ? kNt != 0 : (kD * (kFp8 ? 1U : 2U)) % 128U == 0;
-  static constexpr bool kNarrow = kD == 64 && !kFp8;         // 16-bit rows of 128 bytes
-  static constexpr bool kF8Narrow = kD == 64 && kFp8;        // FP8 rows of 64 bytes
-  static constexpr bool kWide = kD == 256 && !kFp8;          // 16-bit rows of 512 bytes
-  static constexpr bool kF8Wide = kD == 256 && kFp8;         // FP8 rows of 256 bytes
+  static constexpr bool kNtKV = kNt >= 0 ? kNt != 0 : (kD * 2U) % 128U == 0;
+  static constexpr bool kNarrow = kD == 64;  // rows of 128 bytes
+  static constexpr bool kWide = kD == 256;   // rows of 512 bytes
   // Head size 96, 16-bit: rows of 12 chunks (192 bytes). Lanes map to chunks
   // by flat index (16 rows x 12 chunks = 3 DMA instructions per tensor), so a
   // stage holds rows at a 192-byte pitch; a row's chunks are rotated by
@@ -1263,24 +1269,17 @@ struct StreamDecoder {
   // tensor's step rounded up to whole DMA instructions (the spare lanes load
   // a valid chunk into the unused tail), QK over 3 or 4 operand chunks with
   // the chunks past the row read as zero.
-  // FP8 rows at these head sizes (80, 96 or 112 bytes) are kept unrotated
-  // and contiguous in LDS; the converted 16-bit V tile takes the rotated
-  // layout.
   static constexpr bool kRot = kD == 80 || kD == 96 || kD == 112;
-  static constexpr bool kF8Rot = kRot && kFp8;
-  static constexpr uint32_t kRowChunks = kD / 8;               // 16-byte chunks of a 16-bit row
-  static constexpr uint32_t kSrcChunks = kFp8 ? kD / 16 : kD / 8;  // 16-byte chunks of a cache row
-  static constexpr int kRotDma = (kStep * kSrcChunks + 63) / 64;  // DMA instructions per tensor per step
+  static constexpr uint32_t kRowChunks = kD / 8;                  // 16-byte chunks of a row
+  static constexpr int kRotDma = (kStep * kRowChunks + 63) / 64;  // DMA instructions per tensor per step
   // Rotation of row r (in chunks); rot_slot places chunk `chunk` of row r.
   // Head size 96: 2 (r >> 2). Rows r and r + 4 share bank offsets at the
   // 192-byte pitch, and the shift interleaves their 32-byte pieces in the
   // transposed reads (8 rows per pass); measured free of bank conflicts, where
   // 3 (r >> 2) cost 24 cycles per step. Rows of 160 and 224 bytes (head sizes
-  // 80, 112) measured conflict-free unrotated. The FP8 path's converted V
-  // tile stays unrotated: its conversion stores (8 lanes over 128 bytes of
-  // banks at a time) collide in the rotated layout.
+  // 80, 112) measured conflict-free unrotated.
   static __device__ __forceinline__ uint32_t rot_shift(uint32_t r) {
-    return kD == 96 && !kFp8 ? 2U * (r >> 2) : 0U;
+    return kD == 96 ? 2U * (r >> 2) : 0U;
   }
   static __device__ __forceinline__ uint32_t rot_slot(uint32_t r, uint32_t chunk) {
     return (chunk + rot_shift(r)) % kRowChunks;
@@ -1295,29 +1294,19 @@ struct StreamDecoder {
   }
   static constexpr uint32_t kPitch = kD * 2;  // bytes between consecutive tokens' rows in a 16-bit tile
   static constexpr int kDt = kD / 16;         // 16-dim PV tiles
-  // 32-dim QK operand chunks (the last ones zero-padded); FP8 operands pair
-  // them over 64 dims.
-  static constexpr int kKc = kFp8 ? 2 * ((kD + 63) / 64) : (kD + 31) / 32;
+  // 32-dim QK operand chunks (the last ones zero-padded)
+  static constexpr int kKc = (kD + 31) / 32;
   using Ops = MfmaOps<QE>;
   using vec8 = typename Ops::vec8;
   using vec4 = typename Ops::vec4;
-  // PV's element type: the query's for 16-bit caches; F16 for FP8 caches,
-  // whose E4M3 values convert to F16 exactly and whose probabilities then
-  // keep 11 significant bits in one MFMA (BF16 ones need a hi + lo pair).
-  using PvOps = std::conditional_t<kFp8, MfmaOps<F16Elem>, Ops>;
-  using pv8 = typename PvOps::vec8;
-  using pv4 = typename PvOps::vec4;
-  // LDS per wave. 16-bit: kStages stages of [K 4 KiB | V 4 KiB]; PV reads V
-  // in place. FP8: kStages stages of [K bytes 2 KiB | V bytes 2 KiB], then
-  // one 4 KiB tile of the current step's V converted to 16 bits (kVTileOff).
+  // LDS per wave: kStages stages of [K 4 KiB | V 4 KiB]; PV reads V in place.
   static constexpr int kStages = kS;
-  static constexpr uint32_t kF8TileBytes = kRot ? kRotDma * 1024 : kStep * kD;  // FP8 bytes of one tensor's step
-  static constexpr uint32_t kVOff = kRot ? kRotDma * 1024 : kStep * kPitch;  // 16-bit: V within a stage
-  static constexpr uint32_t kStageBytes = kFp8 ? 2 * kF8TileBytes : 2 * kVOff;
-  static constexpr uint32_t kVTileOff = kStages * kStageBytes;  // FP8: converted V tile
-  static constexpr uint32_t kWaveBytes = kStages * kStageBytes + (kFp8 ? kStep * kPitch : 0);
-  static constexpr int kDmaPerStep = kRot ? 2 * kRotDma : kWide ? 16 : kF8Wide ? 8 : kF8Narrow ? 2 : kFp8 || kNarrow ? 4 : 8;
-  static constexpr uint32_t kElem = kFp8 ? 1 : 2;
+  static constexpr uint32_t kVOff = kRot ? kRotDma * 1024 : kStep * kPitch;  // V within a stage
+  static constexpr uint32_t kStageBytes = 2 * kVOff;
+  static constexpr uint32_t kWaveBytes = kStages * kStageBytes;
+  static constexpr int kDmaPerStep = kRot ? 2 * kRotDma : kWide ? 16 : kNarrow ? 4 : 8;
+  static constexpr uint32_t kElem = 2;
+  using Blocks = StepBlocks<1>;
 
   const DecodeArgs& a;
   uint32_t lane, g, c;
@@ -1327,10 +1316,9 @@ struct StreamDecoder {
   const int32_t* table;
   uint64_t kbase, vbase;  // byte address of (block 0, page 0, this kv head)
   uint64_t kstride_b, vstride_b, kstride_p, vstride_p;  // byte strides
-  uint32_t k_voff[4];  // 16-bit: lane's K DMA offset for rows 4i..4i+3
-  uint32_t v_voff[2];  // 16-bit: lane's V DMA offset for even / odd 4-row groups
-  uint32_t f8_k_voff[2], f8_v_voff[2];  // FP8: lane's K / V DMA offsets, rows 8i .. 8i + 7
-  uint32_t w_voff[kWide ? 16 : kF8Wide ? 8 : kRot ? 2 * kRotDma : 1];  // head size 256 / 96: K offsets, then V
+  uint32_t k_voff[4];  // lane's K DMA offset for rows 4i..4i+3 (head size 64: 8i .. 8i + 7)
+  uint32_t v_voff[2];  // lane's V DMA offset for even / odd row groups
+  uint32_t w_voff[kWide ? 16 : kRot ? 2 * kRotDma : 1];  // head size 256 / 80-112: K offsets, then V
   float sl2;
 
   vec8 qb[kHT][kKc];
@@ -1352,17 +1340,22 @@ struct StreamDecoder {
     return static_cast<uint32_t>(((ConstWord*)table)[lb]);
   }
 
+  __device__ __forceinline__ Blocks blocks_of(uint32_t t0) const { return {{block_of(t0)}}; }
+
+  template <int kLater>
+  __device__ __forceinline__ void wait_step(uint32_t later) const {
+    vm_wait_dma_later<kDmaPerStep, kLater>(later);
+  }
+
   __device__ __forceinline__ uint64_t row_base(uint64_t base, uint64_t stride_b, uint64_t stride_p, uint32_t blk,
                                                uint32_t t0) const {
     return base + blk * stride_b + (t0 & (a.block_size - 1U)) * stride_p;
   }
 
-  // Lane DMA offsets. 16-bit K: instruction i brings rows 4i + lane / 16;
+  // Lane DMA offsets. K: instruction i brings rows 4i + lane / 16;
   // row r keeps its 16-byte chunk L at position L ^ (r & 15), so the 16 rows
-  // of one MFMA operand fetch fall in different bank groups. 16-bit V: chunk
-  // L of row r at L ^ 2 (r & 7) (vtile_off). FP8: eight 128-byte rows per
-  // instruction, chunk L of row r at L ^ ((r >> 1) & 7), which keeps the K
-  // operand reads and the V conversion reads bank-conflict free.
+  // of one MFMA operand fetch fall in different bank groups. V: chunk
+  // L of row r at L ^ 2 (r & 7) (vtile_off).
   __device__ __forceinline__ void init_offsets() {
     if constexpr (kRot) {
       // Lane l of instruction i fills LDS chunk 64 i + l = (row, slot); it
@@ -1370,32 +1363,11 @@ struct StreamDecoder {
 #pragma unroll
       for (int i = 0; i < kRotDma; ++i) {
         const uint32_t idx = 64U * i + lane;
-        const bool spare = idx >= kStep * kSrcChunks;  // past the step's rows: reload row 15, chunk 0
-        const uint32_t r = spare ? kStep - 1 : idx / kSrcChunks, slot = spare ? 0U : idx % kSrcChunks;
-        const uint32_t logical = spare || kFp8 ? slot : (slot + kRowChunks - rot_shift(r)) % kRowChunks;
+        const bool spare = idx >= kStep * kRowChunks;  // past the step's rows: reload row 15, chunk 0
+        const uint32_t r = spare ? kStep - 1 : idx / kRowChunks, slot = spare ? 0U : idx % kRowChunks;
+        const uint32_t logical = spare ? slot : (slot + kRowChunks - rot_shift(r)) % kRowChunks;
         w_voff[i] = static_cast<uint32_t>(r * kstride_p) + (logical << 4);
         w_voff[kRotDma + i] = static_cast<uint32_t>(r * vstride_p) + (logical << 4);
-      }
-    } else if constexpr (kF8Narrow) {
-      // FP8 rows of 64 bytes, all 16 rows of a step in one instruction: chunk
-      // L of row r at L ^ ((r >> 2) & 3), so the rows sharing a 256-byte bank
-      // window hold their chunks at distinct offsets.
-      const uint32_t row = lane >> 2;
-      const uint32_t chunk = ((lane & 3U) ^ ((row >> 2) & 3U)) << 4;
-      f8_k_voff[0] = static_cast<uint32_t>(row * kstride_p) + chunk;
-      f8_v_voff[0] = static_cast<uint32_t>(row * vstride_p) + chunk;
-    } else if constexpr (kF8Wide) {
-      // FP8 rows of 256 bytes, four per instruction: chunk L of row r at
-      // L ^ (r & 15) in K and in V (the 8-byte K operand reads of 16 rows,
-      // and the V conversion reads of 16 rows at one chunk, then cover all
-      // banks).
-      const uint32_t row = lane >> 4;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t r = 4 * i + row;
-        const uint32_t chunk = ((lane & 15U) ^ (r & 15U)) << 4;
-        w_voff[i] = static_cast<uint32_t>(row * kstride_p) + chunk;
-        w_voff[4 + i] = static_cast<uint32_t>(row * vstride_p) + chunk;
       }
     } else if constexpr (kWide) {
       // 512-byte rows, two per instruction: K chunk L of row r at L ^ (r & 15),
@@ -1407,23 +1379,15 @@ struct StreamDecoder {
         w_voff[i] = static_cast<uint32_t>(row * kstride_p) + (((lane & 31U) ^ (r & 15U)) << 4);
         w_voff[8 + i] = static_cast<uint32_t>(row * vstride_p) + (((lane & 31U) ^ vtile_swizzle<kPitch>(r)) << 4);
       }
-    } else if (kNarrow) {
-      // 16-bit rows of 128 bytes: K chunk L of row r at L ^ ((r >> 1) & 7)
-      // (as FP8 K), V chunk L at L ^ vtile_swizzle(r).
+    } else if constexpr (kNarrow) {
+      // Rows of 128 bytes: K chunk L of row r at L ^ ((r >> 1) & 7), V chunk L
+      // at L ^ vtile_swizzle(r).
       const uint32_t row = lane >> 3;
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const uint32_t r = 8 * i + row;
-        f8_k_voff[i] = static_cast<uint32_t>(row * kstride_p) + (((lane & 7U) ^ ((r >> 1) & 7U)) << 4);
-        f8_v_voff[i] = static_cast<uint32_t>(row * vstride_p) + (((lane & 7U) ^ vtile_swizzle<kPitch>(r)) << 4);
-      }
-    } else if (kFp8) {
-      const uint32_t row = lane >> 3;
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const uint32_t chunk = ((lane & 7U) ^ (((8 * i + row) >> 1) & 7U)) << 4;
-        f8_k_voff[i] = static_cast<uint32_t>(row * kstride_p) + chunk;
-        f8_v_voff[i] = static_cast<uint32_t>(row * vstride_p) + chunk;
+        k_voff[i] = static_cast<uint32_t>(row * kstride_p) + (((lane & 7U) ^ ((r >> 1) & 7U)) << 4);
+        v_voff[i] = static_cast<uint32_t>(row * vstride_p) + (((lane & 7U) ^ vtile_swizzle<kPitch>(r)) << 4);
       }
     } else {
       const uint32_t row = lane >> 4;
@@ -1437,7 +1401,8 @@ struct StreamDecoder {
   }
 
   // One step's K and V (and nothing else) into a stage.
-  __device__ __forceinline__ void issue(uint8_t* stage, uint32_t blk, uint32_t t0) const {
+  __device__ __forceinline__ void issue(uint8_t* stage, const Blocks& blocks, uint32_t t0) const {
+    const uint32_t blk = blocks.id[0];
     const uint64_t kb = row_base(kbase, kstride_b, kstride_p, blk, t0);
     const uint64_t vb = row_base(vbase, vstride_b, vstride_p, blk, t0);
     if constexpr (kRot) {
@@ -1445,33 +1410,18 @@ struct StreamDecoder {
       for (int i = 0; i < kRotDma; ++i) vm_load16_lds_sv<kNtKV>(w_voff[i], kb, stage + i * 1024);
 #pragma unroll
       for (int i = 0; i < kRotDma; ++i)
-        vm_load16_lds_sv<kNtKV>(w_voff[kRotDma + i], vb, stage + (kFp8 ? kF8TileBytes : kVOff) + i * 1024);
-    } else if constexpr (kF8Narrow) {
-      vm_load16_lds_sv<kNtKV>(f8_k_voff[0], kb, stage);
-      vm_load16_lds_sv<kNtKV>(f8_v_voff[0], vb, stage + kF8TileBytes);
-    } else if constexpr (kF8Wide) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) vm_load16_lds_sv<kNtKV>(w_voff[i], kb + 4 * i * kstride_p, stage + i * 1024);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        vm_load16_lds_sv<kNtKV>(w_voff[4 + i], vb + 4 * i * vstride_p, stage + kF8TileBytes + i * 1024);
+        vm_load16_lds_sv<kNtKV>(w_voff[kRotDma + i], vb, stage + kVOff + i * 1024);
     } else if constexpr (kWide) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) vm_load16_lds_sv<kNtKV>(w_voff[i], kb + 2 * i * kstride_p, stage + i * 1024);
 #pragma unroll
       for (int i = 0; i < 8; ++i) vm_load16_lds_sv<kNtKV>(w_voff[8 + i], vb + 2 * i * vstride_p, stage + kVOff + i * 1024);
-    } else if (kNarrow) {
+    } else if constexpr (kNarrow) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i) vm_load16_lds_sv<kNtKV>(f8_k_voff[i], kb + 8 * i * kstride_p, stage + i * 1024);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        vm_load16_lds_sv<kNtKV>(f8_v_voff[i], vb + 8 * i * vstride_p, stage + kVOff + i * 1024);
-    } else if (kFp8) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i) vm_load16_lds_sv<kNtKV>(f8_k_voff[i], kb + 8 * i * kstride_p, stage + i * 1024);
+      for (int i = 0; i < 2; ++i) vm_load16_lds_sv<kNtKV>(k_voff[i], kb + 8 * i * kstride_p, stage + i * 1024);
 #pragma unroll
       for (int i = 0; i < 2; ++i)
-        vm_load16_lds_sv<kNtKV>(f8_v_voff[i], vb + 8 * i * vstride_p, stage + kF8TileBytes + i * 1024);
+        vm_load16_lds_sv<kNtKV>(v_voff[i], vb + 8 * i * vstride_p, stage + kVOff + i * 1024);
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i) vm_load16_lds_sv<kNtKV>(k_voff[i], kb + 4 * i * kstride_p, stage + i * 1024);
@@ -1480,18 +1430,9 @@ struct StreamDecoder {
     }
   }
 
-  // MFMA A operand kc of token c. 16-bit: dims kc*32 + g*8 .. +7. FP8: dims
-  // (kc >> 1)*64 + g*16 + ((kc ^ g) & 1)*8 .. +7, converted (Q uses the same
-  // dims); the half depends on g so that the two lane groups served together
-  // read different banks.
+  // MFMA A operand kc of token c: dims kc*32 + g*8 .. +7.
   __device__ __forceinline__ vec8 k_operand(const uint8_t* stage, int kc) const {
-    if constexpr (kF8Rot) {
-      const uint32_t chunk = (static_cast<uint32_t>(kc) >> 1) * 4 + g;  // FP8 chunk of 16 dims
-      const uint2 w = *reinterpret_cast<const uint2*>(stage + c * kD + (chunk < kSrcChunks ? chunk : 0U) * 16 +
-                                                      ((kc ^ g) & 1U) * 8);
-      if (chunk >= kSrcChunks) return vec8{};  // dims past the head size
-      return Ops::from_fp8(w.x, w.y);
-    } else if constexpr (kRot) {
+    if constexpr (kRot) {
       const uint32_t chunk = static_cast<uint32_t>(kc) * 4 + g;
       const uint32_t slot = rot_slot(c, chunk < kRowChunks ? chunk : 0U);
       const vec8 k = *reinterpret_cast<const vec8*>(stage + c * kPitch + slot * 16);
@@ -1499,14 +1440,9 @@ struct StreamDecoder {
         if (chunk >= kRowChunks) return vec8{};  // dims past the head size
       }
       return k;
-    } else if (kNarrow) {
+    } else if constexpr (kNarrow) {
       const uint32_t chunk = (static_cast<uint32_t>(kc) * 4 + g) ^ ((c >> 1) & 7U);
       return *reinterpret_cast<const vec8*>(stage + c * kPitch + chunk * 16);
-    } else if (kFp8) {
-      const uint32_t swz = kF8Wide ? (c & 15U) : kF8Narrow ? ((c >> 2) & 3U) : ((c >> 1) & 7U);
-      const uint32_t chunk = ((static_cast<uint32_t>(kc) >> 1) * 4 + g) ^ swz;
-      const uint2 w = *reinterpret_cast<const uint2*>(stage + c * kD + chunk * 16 + ((kc ^ g) & 1U) * 8);
-      return Ops::from_fp8(w.x, w.y);
     } else {
       const uint32_t chunk = (static_cast<uint32_t>(kc) * 4 + g) ^ c;
       return *reinterpret_cast<const vec8*>(stage + c * kPitch + chunk * 16);
@@ -1527,7 +1463,7 @@ struct StreamDecoder {
     u32x4 qw[kHT][kKc];
     uint32_t dim[kKc];  // this lane's eight dims of chunk kc
 #pragma unroll
-    for (int kc = 0; kc < kKc; ++kc) dim[kc] = kFp8 ? ((kc >> 1) * 64 + g * 16 + ((kc ^ g) & 1U) * 8) : (kc * 32 + g * 8);
+    for (int kc = 0; kc < kKc; ++kc) dim[kc] = kc * 32 + g * 8;
 #pragma unroll
     for (int ht = 0; ht < kHT; ++ht) {
       const uint32_t h = min(ht * 16U + c, live - 1U);  // rows past the group are zeroed below
@@ -1563,61 +1499,11 @@ struct StreamDecoder {
     }
   }
 
-  // FP8 V bytes of a stage -> the wave's swizzled 16-bit V tile (rows past
-  // the sequence end become zero). Head sizes 64 and 128: lane handles kD / 4
-  // bytes of token lane >> 2; head size 256: lane handles four 16-byte chunks
-  // of token lane & 15. 16-byte LDS reads are served 16 lanes at a time over 256 bytes
-  // of banks, 16-byte writes 8 lanes at a time over 128 bytes; the row
-  // mapping, the V swizzle and the order of each lane's two stores (the
-  // `up` lanes store the upper 16-bit chunk first) keep every read and every
-  // store free of bank conflicts.
-  __device__ __forceinline__ void stage_v_fp8(const uint8_t* stage, uint8_t* tile, uint32_t t0) const {
-    if constexpr (kF8Rot) {
-      // Rows of 5, 6 or 7 FP8 chunks: lanes take chunks by flat index.
-#pragma unroll
-      for (uint32_t it = 0; it < (kStep * kSrcChunks + 63) / 64; ++it) {
-        const uint32_t idx = it * 64U + lane;
-        if (idx < kStep * kSrcChunks) {
-          const uint32_t t = idx / kSrcChunks, lc = idx % kSrcChunks;
-          const u32x4 raw = *reinterpret_cast<const u32x4*>(stage + kF8TileBytes + t * kD + lc * 16);
-          const u32x4 w = t0 + t < len ? raw : u32x4{0U, 0U, 0U, 0U};
-          const pv8 lo = PvOps::from_fp8(w[0], w[1]), hi = PvOps::from_fp8(w[2], w[3]);
-          // Lanes 4..7 of each eight store their upper chunk first, which
-          // spreads each store's eight lanes over distinct bank quarters.
-          const uint32_t up = (lane >> 2) & 1U;
-          *reinterpret_cast<pv8*>(tile + vt_off(t, 2 * lc + up)) = up ? hi : lo;
-          *reinterpret_cast<pv8*>(tile + vt_off(t, 2 * lc + 1 - up)) = up ? lo : hi;
-        }
-      }
-      return;
-    }
-    constexpr uint32_t kLaneChunks = kD / 64;  // 16-byte FP8 chunks per lane
-    const uint32_t t = kF8Wide ? (lane & 15U) : (lane >> 2);
-    const uint32_t q = kF8Wide ? (lane >> 4) : (lane & 3U);
-    const bool live = t0 + t < len;
-    const uint8_t* vrow = stage + kF8TileBytes + t * kD;
-    const uint32_t up = kF8Wide ? ((t >> 2) & 1U) : kF8Narrow ? (lane & 1U) : ((lane >> 1) & 1U);
-    const uint32_t swz = kF8Wide ? (t & 15U) : kF8Narrow ? ((t >> 2) & 3U) : ((t >> 1) & 7U);
-#pragma unroll
-    for (uint32_t h = 0; h < kLaneChunks; ++h) {
-      // Logical 16-byte chunk of the FP8 row: head size 256 interleaves the
-      // four lane groups (q, q + 4, q + 8, q + 12), which measured free of
-      // read conflicts where q * 4 + h read 16 conflict cycles per step.
-      const uint32_t lc = kF8Wide ? q + 4U * h : q * kLaneChunks + h;
-      const u32x4 raw = *reinterpret_cast<const u32x4*>(vrow + ((lc ^ swz) << 4));
-      const u32x4 w = live ? raw : u32x4{0U, 0U, 0U, 0U};
-      // 16-bit chunks 2 lc and 2 lc + 1 (8 dims each).
-      const pv8 lo = PvOps::from_fp8(w[0], w[1]), hi = PvOps::from_fp8(w[2], w[3]);
-      const uint32_t ch = lc * 2;
-      *reinterpret_cast<pv8*>(tile + vtile_off<kPitch>(t, ch + up)) = up ? hi : lo;
-      *reinterpret_cast<pv8*>(tile + vtile_off<kPitch>(t, ch + 1 - up)) = up ? lo : hi;
-    }
-  }
-
   // Tile rows of tokens past the sequence end (possible only in its last
   // step) may hold unwritten cache slots: zero them so P = 0 meets a finite V.
-  __device__ __forceinline__ void zero_dead_rows(uint8_t* tile, uint32_t t0) const {
+  __device__ __forceinline__ void zero_dead_rows(uint8_t* stage, uint32_t t0) const {
     if (t0 + kStep <= len) return;  // uniform
+    uint8_t* tile = stage + kVOff;
     const uint32_t t = lane >> 2;   // 4 lanes per row, kPitch / 4 bytes each
     if (t0 + t >= len) {
       uint8_t* part = tile + t * kPitch + (lane & 3U) * (kPitch / 4);
@@ -1633,9 +1519,16 @@ struct StreamDecoder {
     }
   }
 
+  // One step of a stage whose loads have arrived.
+  __device__ __forceinline__ void consume(const uint8_t* stage, uint32_t t0) {
+    f32x4 s[kHT];
+    qk(stage, s);
+    softmax_pv(s, t0, stage + kVOff);
+  }
+
   __device__ __forceinline__ void softmax_pv(f32x4 (&s)[kHT], uint32_t t0, const uint8_t* tile) {
     typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-    pv4 pb[kHT], pr[kHT];
+    vec4 pb[kHT], pr[kHT];
 #pragma unroll
     for (int ht = 0; ht < kHT; ++ht) {
 #pragma unroll
@@ -1660,10 +1553,10 @@ struct StreamDecoder {
         p[r] = __builtin_amdgcn_exp2f(s[ht][r] - m[ht]);
         lsum[ht] += p[r];
       }
-      const uint32_t w0 = PvOps::pack2(p[0], p[1]), w1 = PvOps::pack2(p[2], p[3]);
-      pb[ht] = __builtin_bit_cast(pv4, u32x2{w0, w1});
-      if constexpr (PvOps::kSplitP)
-        pr[ht] = __builtin_bit_cast(pv4, u32x2{PvOps::rest2(p[0], p[1], w0), PvOps::rest2(p[2], p[3], w1)});
+      const uint32_t w0 = Ops::pack2(p[0], p[1]), w1 = Ops::pack2(p[2], p[3]);
+      pb[ht] = __builtin_bit_cast(vec4, u32x2{w0, w1});
+      if constexpr (Ops::kSplitP)
+        pr[ht] = __builtin_bit_cast(vec4, u32x2{Ops::rest2(p[0], p[1], w0), Ops::rest2(p[2], p[3], w1)});
     }
     const uint32_t k = c >> 2, q = c & 3U;
     lds_u8* base = (lds_u8*)tile;
@@ -1673,7 +1566,7 @@ struct StreamDecoder {
       const s16x4 va = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(base + off));
 #pragma unroll
       for (int ht = 0; ht < kHT; ++ht) {
-        if constexpr (PvOps::kSplitP) {
+        if constexpr (Ops::kSplitP) {
           // One K = 32 MFMA: K index 8g + r pairs token 4g + r with hi, 8g + 4 + r
           // with its remainder lo; the V operand repeats the lane's four tokens.
           typedef short s16x8 __attribute__((ext_vector_type(8)));
@@ -1681,9 +1574,9 @@ struct StreamDecoder {
           const s16x4 h4 = __builtin_bit_cast(s16x4, pb[ht]), l4 = __builtin_bit_cast(s16x4, pr[ht]);
           const s16x8 a8 = __builtin_shufflevector(v4, v4, 0, 1, 2, 3, 0, 1, 2, 3);
           const s16x8 b8 = __builtin_shufflevector(h4, l4, 0, 1, 2, 3, 4, 5, 6, 7);
-          acc[ht][dt] = PvOps::mma(__builtin_bit_cast(pv8, a8), __builtin_bit_cast(pv8, b8), acc[ht][dt]);
+          acc[ht][dt] = Ops::mma(__builtin_bit_cast(vec8, a8), __builtin_bit_cast(vec8, b8), acc[ht][dt]);
         } else {
-          acc[ht][dt] = PvOps::mma16(__builtin_bit_cast(pv4, va), pb[ht], acc[ht][dt]);
+          acc[ht][dt] = Ops::mma16(__builtin_bit_cast(vec4, va), pb[ht], acc[ht][dt]);
         }
       }
     }
@@ -1712,6 +1605,8 @@ struct F32StreamDecoder {
   static_assert(kD % 16 == 0 && kD >= 64 && kD <= 128, "whole 16-dim tiles");
   static constexpr bool kNtKV = kNt >= 0 ? kNt != 0 : (kD * 4U) % 128U == 0;
   static constexpr int kHT = 1;
+  static constexpr uint32_t kTok = kStep;
+  using Blocks = StepBlocks<1>;
   static constexpr int kDt = kD / 16;                 // accumulator tiles
   static constexpr int kKc = kD / 16;                 // 16-dim QK chunks of a lane group
   static constexpr uint32_t kPitch = kD * 4;          // bytes of a row
@@ -1722,7 +1617,6 @@ struct F32StreamDecoder {
   static constexpr int kStages = kS;
   static constexpr uint32_t kVOff = kStep * kPitch;
   static constexpr uint32_t kStageBytes = 2 * kVOff;
-  static constexpr uint32_t kVTileOff = 0;            // PV reads V in place
   static constexpr uint32_t kWaveBytes = kStages * kStageBytes;
   static constexpr int kDmaPerStep = 2 * kDma;
   static constexpr uint32_t kElem = 4;
@@ -1756,6 +1650,13 @@ struct F32StreamDecoder {
     return static_cast<uint32_t>(((ConstWord*)table)[lb]);
   }
 
+  __device__ __forceinline__ Blocks blocks_of(uint32_t t0) const { return {{block_of(t0)}}; }
+
+  template <int kLater>
+  __device__ __forceinline__ void wait_step(uint32_t later) const {
+    vm_wait_dma_later<kDmaPerStep, kLater>(later);
+  }
+
   __device__ __forceinline__ uint64_t row_base(uint64_t base, uint64_t stride_b, uint64_t stride_p, uint32_t blk,
                                                uint32_t t0) const {
     return base + blk * stride_b + (t0 & (a.block_size - 1U)) * stride_p;
@@ -1776,7 +1677,8 @@ struct F32StreamDecoder {
       k_off[kc] = c * kPitch + ((4U * kc + g + (c >> kRotShift)) % kRowChunks) * 16U;
   }
 
-  __device__ __forceinline__ void issue(uint8_t* stage, uint32_t blk, uint32_t t0) const {
+  __device__ __forceinline__ void issue(uint8_t* stage, const Blocks& blocks, uint32_t t0) const {
+    const uint32_t blk = blocks.id[0];
     const uint64_t kb = row_base(kbase, kstride_b, kstride_p, blk, t0);
     const uint64_t vb = row_base(vbase, vstride_b, vstride_p, blk, t0);
 #pragma unroll
@@ -1812,8 +1714,9 @@ struct F32StreamDecoder {
 
   // Rows of tokens past the sequence end (possible only in its last step):
   // zeroed so that P = 0 meets a finite V. A quarter wave per row.
-  __device__ __forceinline__ void zero_dead_rows(uint8_t* tile, uint32_t t0) const {
+  __device__ __forceinline__ void zero_dead_rows(uint8_t* stage, uint32_t t0) const {
     if (t0 + kStep <= len) return;  // uniform
+    uint8_t* tile = stage + kVOff;
 #pragma unroll
     for (uint32_t r = 0; r < 4; ++r) {
       if (t0 + 4 * g + r >= len) {
@@ -1824,6 +1727,12 @@ struct F32StreamDecoder {
         }
       }
     }
+  }
+
+  __device__ __forceinline__ void consume(const uint8_t* stage, uint32_t t0) {
+    f32x4 s[1];
+    qk(stage, s);
+    softmax_pv(s, t0, stage + kVOff);
   }
 
   // PV tiles of kE elements per lane from dim kBase on: tile (j) row i is dim
@@ -1891,9 +1800,268 @@ struct F32StreamDecoder {
   }
 };
 
+// 16-bit queries over FP8 caches. A step is 32 tokens, two halves of 16 rows
+// (a half lies in one block): K = 32 fills PV's MFMA with FP8 V read straight
+// from the stage. Bound by VALU issue next to HBM: FP8 rows move half the bytes
+// per score, and every byte is converted once (v_cvt_scalef32_pk, two values
+// each). The previous form staged V as F16 in an LDS tile per 16-token step
+// (16 conversions, 24 selects, 4 stores and 8 reads per lane) and padded QK to
+// whole 64 dims. Decode calls us, before -> now: 32/32 heads, head size 96, 32
+// ragged sequences NHD 113 -> 100; 64 sequences, Hq 32 / Hkv 8, 0.27-0.54 GB of HND
+// cache: 64 81.9 -> 77.3, 80 115 -> 79.3, 96 107 -> 81.6, 112 83.5 -> 79.0, 128
+// 90.8 -> 79.8, 256 100 -> 84; 48/1 x 16k 83 -> 65; 32/1 x 64k-128k 66.6 -> 49.8.
+//   S: as StreamDecoder, K converted as it is read; half b's scores of tokens
+//      4g + r, r = 0 .. 3, land in lane (g, c).
+//   PV: one ds_read_b64_tr_b8 per 16 dims brings lane (g, c) dim c of eight
+//      tokens, rows 4g .. 4g + 3 of both halves, which is the order that the
+//      lane's eight probabilities are in: K index 8g + 4b + r is token 4g + r
+//      of half b. V becomes F16 (exact for E4M3; the probabilities keep 11
+//      significant bits in one MFMA, where BF16 ones need a hi + lo pair).
+template <typename QE, int kHTiles, uint32_t kD, int kS = kStreamStages, int kNt = -1>
+struct Fp8StreamDecoder {
+  static_assert(kD == kDim || kD == 64 || ((kD == 80 || kD == 96 || kD == 112 || kD == 256) && kHTiles == 1),
+                "head size 64, 128, or 80 / 96 / 112 / 256 with one head tile");
+  static constexpr int kHT = kHTiles;
+  static constexpr uint32_t kTok = 2 * kStep;
+  static constexpr uint32_t kElem = 1;
+  using Blocks = StepBlocks<2>;
+  // Non-temporal hint: see StreamDecoder::kNtKV.
+  static constexpr bool kNtKV = kNt >= 0 ? kNt != 0 : kD % 128U == 0;
+  static constexpr int kDt = kD / 16;  // 16-dim PV tiles
+  // QK operand chunks of 32 dims: pairs over 64 dims, then the rest.
+  static constexpr int kPairs = 2 * (kD / 64);
+  static constexpr int kKc = kPairs + (kD % 64 + 31) / 32;
+  static constexpr uint32_t kChunks = kD / 16;         // 16-byte chunks of a row
+  static constexpr bool kSwz = (kChunks & (kChunks - 1)) == 0;
+  static constexpr uint32_t kHalfBytes = kStep * kD;   // 16 rows of one tensor
+  static constexpr int kDma = (kHalfBytes + 1023) / 1024;  // DMA instructions per tensor and half
+  // Active lanes of the last of them (rows of 80-112 bytes fill no whole number).
+  static constexpr uint32_t kTailLanes = kHalfBytes % 1024 == 0 ? 64U : kHalfBytes % 1024 / 16;
+  static constexpr int kDmaPerHalf = 2 * kDma;
+  // A stage: K of both halves, then V of both. Unswizzled V rows (80-112
+  // bytes) put half 1 where its eight rows of a transposed read fall on the
+  // 16-byte bank slots that half 0's leave free.
+  static constexpr uint32_t kVOff = 2 * kHalfBytes;
+  static constexpr uint32_t kVOff1 = 3 * kHalfBytes + (kSwz ? 0U : kD == 96 ? 16U : 128U);
+  static constexpr int kStages = kS;
+  static constexpr uint32_t kStageBytes = kVOff1 + kHalfBytes;
+  static constexpr uint32_t kWaveBytes = kStages * kStageBytes;
+  using Ops = MfmaOps<QE>;
+  using vec8 = typename Ops::vec8;
+  using PvOps = MfmaOps<F16Elem>;
+  using pv8 = typename PvOps::vec8;
+
+  const DecodeArgs& a;
+  uint32_t lane, g, c;
+  uint32_t p1;
+  uint32_t len;
+  uint32_t last_block;
+  uint32_t odd;  // 1 when the wave's last step has only half 0
+  const int32_t* table;
+  uint64_t kbase, vbase;
+  uint64_t kstride_b, vstride_b, kstride_p, vstride_p;
+  uint32_t k_voff[kDma], v_voff[kDma], v1_voff[kSwz ? kDma : 1];  // lane's DMA offsets (V: half 0, half 1)
+  uint32_t v_off;  // lane's place in a stage for the transposed V reads (dims 0 .. 15)
+  float sl2;
+
+  vec8 qb[kHT][kKc];
+  f32x4 acc[kHT][kDt];
+  float m[kHT];
+  float lsum[kHT];
+
+  __device__ __forceinline__ Fp8StreamDecoder(const DecodeArgs& args) : a(args) {}
+
+  __device__ __forceinline__ uint32_t block_of(uint32_t t0) const {
+    const uint32_t lb = min(t0 >> a.block_shift, last_block);
+    using ConstWord = const __attribute__((address_space(4))) int32_t;
+    return static_cast<uint32_t>(((ConstWord*)table)[lb]);
+  }
+
+  __device__ __forceinline__ Blocks blocks_of(uint32_t t0) const { return {{block_of(t0), block_of(t0 + kStep)}}; }
+
+  // Waits for a step's DMA, counted in halves: a last step without half 1
+  // issued half the loads.
+  template <int kLater>
+  __device__ __forceinline__ void wait_step(uint32_t later) const {
+    vm_wait_dma_later<kDmaPerHalf, 2 * kLater>(later == 0 ? 0U : 2 * later - odd);
+  }
+
+  // Chunk L of row r sits at L ^ k_swizzle(r) in K, L ^ v_swizzle(b, r) in V
+  // of half b: the 8-byte K operand reads of 16 rows, and the transposed reads
+  // of eight rows of both halves, then cover distinct banks.
+  static __device__ __forceinline__ uint32_t k_swizzle(uint32_t r) {
+    return kD == 256 ? (r & 15U) : kD == 128 ? ((r >> 1) & 7U) : kD == 64 ? ((r >> 2) & 3U) : 0U;
+  }
+  static __device__ __forceinline__ uint32_t v_swizzle(uint32_t b, uint32_t r) {
+    return kSwz ? k_swizzle(r) ^ (b * (kChunks / 2)) : 0U;
+  }
+
+  __device__ __forceinline__ void init_offsets() {
+#pragma unroll
+    for (int i = 0; i < kDma; ++i) {
+      const uint32_t idx = min(64U * i + lane, kStep * kChunks - 1U);  // lanes past the tail are not active there
+      const uint32_t r = idx / kChunks, slot = idx % kChunks;
+      k_voff[i] = static_cast<uint32_t>(r * kstride_p) + ((slot ^ k_swizzle(r)) << 4);
+      v_voff[i] = static_cast<uint32_t>(r * vstride_p) + ((slot ^ v_swizzle(0, r)) << 4);
+      if constexpr (kSwz) v1_voff[i] = static_cast<uint32_t>(r * vstride_p) + ((slot ^ v_swizzle(1, r)) << 4);
+    }
+    const uint32_t b = c >> 3, r = 4 * g + ((c >> 1) & 3U);  // row of this lane's transposed reads
+    v_off = (b != 0 ? kVOff1 : kVOff) + r * kD + (v_swizzle(b, r) << 4) + (c & 1U) * 8;
+  }
+
+  template <int kB>
+  __device__ __forceinline__ void issue_half(uint8_t* stage, uint32_t blk, uint32_t t0) const {
+    const uint64_t in_block = t0 & (a.block_size - 1U);
+    const uint64_t kb = kbase + blk * kstride_b + in_block * kstride_p;
+    const uint64_t vb = vbase + blk * vstride_b + in_block * vstride_p;
+    uint8_t* kt = stage + kB * kHalfBytes;
+    uint8_t* vt = stage + (kB == 0 ? kVOff : kVOff1);
+    auto pair = [&](int i) {
+      vm_load16_lds_sv<kNtKV>(k_voff[i], kb, kt + i * 1024);
+      vm_load16_lds_sv<kNtKV>(kSwz && kB == 1 ? v1_voff[i] : v_voff[i], vb, vt + i * 1024);
+    };
+#pragma unroll
+    for (int i = 0; i + 1 < kDma; ++i) pair(i);
+    if (kTailLanes == 64U || lane < kTailLanes) pair(kDma - 1);
+  }
+
+  // One step's K and V (and nothing else) into a stage.
+  __device__ __forceinline__ void issue(uint8_t* stage, const Blocks& blocks, uint32_t t0) const {
+    issue_half<0>(stage, blocks.id[0], t0);
+    if (t0 + kStep < p1) issue_half<1>(stage, blocks.id[1], t0 + kStep);  // uniform
+  }
+
+  template <typename F>
+  __device__ __forceinline__ void each_dims4(int ht, F&& f) const {
+#pragma unroll
+    for (int dt = 0; dt < kDt; ++dt) f(dt * 16U + 4U * g, acc[ht][dt]);
+  }
+
+  // The eight dims of operand chunk kc in this lane group (past the head size
+  // for some groups of the last chunk). In a pair the half of the FP8 chunk
+  // depends on g, so that the two lane groups served together read different
+  // banks.
+  __device__ __forceinline__ uint32_t chunk_dim(int kc) const {
+    return kc < kPairs ? (kc >> 1) * 64 + g * 16 + ((kc ^ g) & 1U) * 8 : (kD & ~63U) + (kc - kPairs) * 32 + g * 8;
+  }
+
+  __device__ __forceinline__ void load_query(uint32_t seq, uint32_t head0, uint32_t live) {
+    u32x4 qw[kHT][kKc];
+#pragma unroll
+    for (int ht = 0; ht < kHT; ++ht) {
+      const uint32_t h = min(ht * 16U + c, live - 1U);  // rows past the group are zeroed below
+      const uint16_t* qrow =
+          static_cast<const uint16_t*>(a.query) + (static_cast<uint64_t>(seq) * a.query_heads + head0 + h) * kD;
+#pragma unroll
+      for (int kc = 0; kc < kKc; ++kc)
+        qw[ht][kc] = *reinterpret_cast<const u32x4*>(qrow + (chunk_dim(kc) < kD ? chunk_dim(kc) : 0U));
+    }
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+#pragma unroll
+    for (int ht = 0; ht < kHT; ++ht) {
+#pragma unroll
+      for (int kc = 0; kc < kKc; ++kc)
+        qb[ht][kc] = __builtin_bit_cast(
+            vec8, ht * 16U + c < live && chunk_dim(kc) < kD ? qw[ht][kc] : u32x4{0U, 0U, 0U, 0U});
+    }
+  }
+
+  // MFMA A operand kc of row c. Lanes past the head size read the row's first
+  // dims and meet zero query dims: E4M3 has no infinity, and a NaN among them
+  // makes the score NaN by itself.
+  __device__ __forceinline__ vec8 k_operand(const uint8_t* tile, int kc) const {
+    const uint32_t dim = chunk_dim(kc);
+    uint32_t off;
+    if constexpr (kSwz) {
+      off = (((static_cast<uint32_t>(kc) >> 1) * 4 + g) ^ k_swizzle(c)) * 16 + ((kc ^ g) & 1U) * 8;
+    } else {
+      off = dim < kD ? dim : 0U;
+    }
+    const uint2 w = *reinterpret_cast<const uint2*>(tile + c * kD + off);
+    return Ops::from_fp8(w.x, w.y);
+  }
+
+  // V rows past the partition's end (possible only in its last step; they may
+  // hold unwritten cache slots, or nothing was loaded): zeroed so that P = 0
+  // meets a finite V. Two lanes per row.
+  __device__ __forceinline__ void zero_dead_rows(uint8_t* stage, uint32_t t0) const {
+    if (t0 + kTok <= p1) return;  // uniform
+    const uint32_t row = lane >> 1;
+    if (t0 + row >= p1) {
+      uint2* dst = reinterpret_cast<uint2*>(stage + (row < kStep ? kVOff : kVOff1) + (row & 15U) * kD +
+                                            (lane & 1U) * (kD / 2));
+#pragma unroll
+      for (uint32_t i = 0; i < kD / 16; ++i) dst[i] = make_uint2(0U, 0U);
+    }
+  }
+
+  // One step of a stage whose loads have arrived.
+  __device__ __forceinline__ void consume(const uint8_t* stage, uint32_t t0) {
+    f32x4 s[kHT][2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      vec8 kop[kKc];
+#pragma unroll
+      for (int kc = 0; kc < kKc; ++kc) kop[kc] = k_operand(stage + b * kHalfBytes, kc);
+#pragma unroll
+      for (int ht = 0; ht < kHT; ++ht) {
+        s[ht][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int kc = 0; kc < kKc; ++kc) s[ht][b] = Ops::mma(kop[kc], qb[ht][kc], s[ht][b]);
+      }
+    }
+    const bool tail = t0 + kTok > p1;  // uniform: only a partition's last step holds tokens past its end
+    pv8 pb[kHT];
+#pragma unroll
+    for (int ht = 0; ht < kHT; ++ht) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[ht][b][r] *= sl2;
+      }
+      if (tail) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) s[ht][b][r] = t0 + b * kStep + 4 * g + r < p1 ? s[ht][b][r] : -INFINITY;
+        }
+      }
+      const f32x4 &x = s[ht][0], &y = s[ht][1];
+      const float cmax = head_max(fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])),
+                                        fmaxf(fmaxf(y[0], y[1]), fmaxf(y[2], y[3]))));
+      const float mn = fmaxf(m[ht], cmax);  // finite: every step has a valid token
+      // Rescale only when some head's maximum moved (exact; usually skipped).
+      if (__builtin_amdgcn_ballot_w64(mn > m[ht]) != 0) {
+        const float alpha = __builtin_amdgcn_exp2f(m[ht] - mn);
+        lsum[ht] *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < kDt; ++dt) acc[ht][dt] *= alpha;
+        m[ht] = mn;
+      }
+      float p[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) p[j] = __builtin_amdgcn_exp2f(s[ht][j >> 2][j & 3] - m[ht]);
+      lsum[ht] += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+      pb[ht] = __builtin_bit_cast(pv8, u32x4{PvOps::pack2(p[0], p[1]), PvOps::pack2(p[2], p[3]),
+                                             PvOps::pack2(p[4], p[5]), PvOps::pack2(p[6], p[7])});
+    }
+    typedef int i32x2 __attribute__((ext_vector_type(2)));
+    typedef __attribute__((address_space(3))) i32x2 lds_i32x2;
+    lds_u8* base = (lds_u8*)stage;
+#pragma unroll
+    for (uint32_t dt = 0; dt < kDt; ++dt) {
+      const uint32_t off = kSwz ? v_off ^ (dt << 4) : v_off + (dt << 4);
+      const i32x2 w = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_i32x2*)(base + off));
+      const pv8 va = PvOps::from_fp8(static_cast<uint32_t>(w[0]), static_cast<uint32_t>(w[1]));
+#pragma unroll
+      for (int ht = 0; ht < kHT; ++ht) acc[ht][dt] = PvOps::mma(va, pb[ht], acc[ht][dt]);
+    }
+  }
+};
+
 template <typename QE, bool kFp8, int kHT, uint32_t kD, int kS, int kNt>
 struct DecoderOf {
-  using type = StreamDecoder<QE, kFp8, kHT, kD, kS, kNt>;
+  using type = std::conditional_t<kFp8, Fp8StreamDecoder<QE, kHT, kD, kS, kNt>, StreamDecoder<QE, kHT, kD, kS, kNt>>;
 };
 template <uint32_t kD, int kS, int kNt>
 struct DecoderOf<F32Elem, false, 1, kD, kS, kNt> {
@@ -2308,10 +2476,11 @@ __device__ __forceinline__ void pair_combine(const uint8_t* tile, float& m, floa
 // each); after the step loop the same memory holds each wave's O (16 heads x
 // 128 dims F32 = 8 KiB) for the cross-wave reduction.
 template <typename QE, bool kFp8, int kSplit, int kHT = 1, uint32_t kD = kDim,
-          int kS = kFp8 ? kStreamStagesFp8 : kStreamStages, int kNt = -1, bool kPair = false>
+          int kS = kStreamStages, int kNt = -1, bool kPair = false>
 __device__ __forceinline__ void stream_item(const DecodeArgs& a, uint8_t* tiles, const WorkItem& item,
                                             bool preloaded = false, const uint32_t* first_blocks = nullptr,
                                             uint8_t* partner = nullptr) {
+  constexpr bool kPreload = !kFp8;  // direct_item loads one block per step
   static_assert(kHT == 1 || kSplit == 1, "two head tiles run one wave per item");
   using Dec = Decoder<QE, kFp8, kHT, kD, kS, kNt>;
   constexpr int S = Dec::kStages;
@@ -2349,14 +2518,16 @@ __device__ __forceinline__ void stream_item(const DecodeArgs& a, uint8_t* tiles,
   }
   dec.sl2 = a.score_scale_log2 * k_scale;
 
-  // Steps of this partition: step k covers [p0 + 16k, p0 + 16k + 16); wave
-  // w takes steps w, w + kSplit, ... Block-table reads past the wave's last
+  // Steps of this partition: step k covers Dec::kTok tokens from p0 + k kTok;
+  // wave w takes steps w, w + kSplit, ... Block-table reads past the wave's last
   // step are clamped onto it; no K/V load is issued past it.
-  const uint32_t nst = (dec.p1 - p0 + kStep - 1) / kStep;
+  constexpr uint32_t kTok = Dec::kTok;
+  const uint32_t nst = (dec.p1 - p0 + kTok - 1) / kTok;
   const uint32_t my_n = nst > wave ? (nst - wave + kSplit - 1) / kSplit : 0;
-  const uint32_t st = kSplit * kStep;
-  const uint32_t t_first = p0 + wave * kStep;
+  const uint32_t st = kSplit * kTok;
+  const uint32_t t_first = p0 + wave * kTok;
   const uint32_t t_last = t_first + (my_n > 0 ? my_n - 1 : 0) * st;
+  if constexpr (kFp8) dec.odd = t_last + kStep >= dec.p1 ? 1U : 0U;
 
 #pragma unroll
   for (int ht = 0; ht < kHT; ++ht) {
@@ -2369,25 +2540,30 @@ __device__ __forceinline__ void stream_item(const DecodeArgs& a, uint8_t* tiles,
   if (my_n > 0) {
     // Block IDs run S steps ahead of the loads that use them.
     uint8_t* tl[S];
-    uint32_t nx[S];
-    uint32_t bk[S];
+    typename Dec::Blocks nx[S];
+    typename Dec::Blocks bk[S];
 #pragma unroll
     for (int i = 0; i < S; ++i) tl[i] = tw + i * Dec::kStageBytes;
-    if (preloaded) {
-      // The block IDs of steps 0 .. 2S - 1, loaded with the item's length.
+    bool loaded = false;
+    if constexpr (kPreload) {
+      if (preloaded) {
+        // The block IDs of steps 0 .. 2S - 1, loaded with the item's length.
 #pragma unroll
-      for (int i = 0; i < S; ++i) {
-        bk[i] = first_blocks[i];
-        nx[i] = first_blocks[S + i];
+        for (int i = 0; i < S; ++i) {
+          bk[i].id[0] = first_blocks[i];
+          nx[i].id[0] = first_blocks[S + i];
+        }
+        loaded = true;
       }
-    } else {
+    }
+    if (!loaded) {
 #pragma unroll
-      for (int i = 0; i < S; ++i) bk[i] = dec.block_of(min(t_first + i * st, t_last));
+      for (int i = 0; i < S; ++i) bk[i] = dec.blocks_of(min(t_first + i * st, t_last));
 #pragma unroll
-      for (int i = 0; i < S; ++i) nx[i] = dec.block_of(min(t_first + (S + i) * st, t_last));
+      for (int i = 0; i < S; ++i) nx[i] = dec.blocks_of(min(t_first + (S + i) * st, t_last));
     }
 #pragma unroll
-    for (int i = 0; i < S; ++i) scalar_ready(bk[i]);
+    for (int i = 0; i < S; ++i) bk[i].ready();
 #pragma unroll
     for (int i = 0; i < S; ++i) {
       if (i < my_n) dec.issue(tl[i], bk[i], t_first + i * st);
@@ -2402,25 +2578,18 @@ __device__ __forceinline__ void stream_item(const DecodeArgs& a, uint8_t* tiles,
       for (int i = 0; i < S; ++i) {
         if (n + i < my_n) {
           const uint32_t t0 = t_first + (n + i) * st;
-          uint8_t* vtile = kFp8 ? tw + Dec::kVTileOff : tl[i] + Dec::kVOff;
           // this step's loads; the later steps' (up to S - 1) stay in flight
-          LOOM_WAVE_STALL(n + i, my_n, (vm_wait_dma_later<Dec::kDmaPerStep, S - 1>(my_n - 1 - (n + i))));
-          scalar_ready(nx[i]);
-          if constexpr (kFp8) {
-            dec.stage_v_fp8(tl[i], vtile, t0);
-          } else {
-            dec.zero_dead_rows(vtile, t0);
-          }
+          LOOM_WAVE_STALL(n + i, my_n, (dec.template wait_step<S - 1>(my_n - 1 - (n + i))));
+          nx[i].ready();
+          dec.zero_dead_rows(tl[i], t0);
           wave_fence_lds();
-          f32x4 sc[kHT];
-          dec.qk(tl[i], sc);
-          dec.softmax_pv(sc, t0, vtile);
+          dec.consume(tl[i], t0);
           wait_lds_reads();
           // No load past the item's last step: such a load would re-read
           // rows nobody consumes, and the wave's exit would wait for it.
           if (n + i + S < my_n) dec.issue(tl[i], nx[i], t0 + S * st);
           wave_fence_lds();
-          nx[i] = dec.block_of(min(t0 + 2 * S * st, t_last));
+          nx[i] = dec.blocks_of(min(t0 + 2 * S * st, t_last));
         }
       }
     }
@@ -2507,9 +2676,12 @@ __device__ __forceinline__ void stream_item(const DecodeArgs& a, uint8_t* tiles,
 // the clobber keeps the compiler from moving LDS accesses across it.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory"); }
 
-// Pipeline stages shared by the waves of a wide-group workgroup (16-bit: 8 KiB
-// each; FP8: 4 KiB, plus one converted V tile per wave).
+// Pipeline stages shared by the waves of a wide-group workgroup (8 KiB each at
+// head size 128). FP8 stages hold 32 tokens; three of them leave six
+// workgroups per CU where four leave five (48/1 x 16k, 1,536 items: 71.2 ->
+// 64.6 us; every other FP8 group 1-2% faster).
 constexpr int kSharedStages = 4;
+constexpr int kSharedStagesFp8 = 3;
 
 // One work item of a group of 33-128 query heads: kWaves waves, wave w
 // computing heads 32 w .. 32 w + 31 with two head tiles, from a ring of K/V
@@ -2520,8 +2692,9 @@ constexpr int kSharedStages = 4;
 // steps, so all of them reach every barrier.
 template <typename QE, bool kFp8, int kWaves, uint32_t kD, int kHTW = 2>
 __device__ __forceinline__ void stream_item_shared(const DecodeArgs& a, uint8_t* tiles, const WorkItem& item) {
-  using Dec = StreamDecoder<QE, kFp8, kHTW, kD>;
-  constexpr int S = kSharedStages;
+  constexpr int S = kFp8 ? kSharedStagesFp8 : kSharedStages;
+  using Dec = Decoder<QE, kFp8, kHTW, kD, S, -1>;
+  constexpr uint32_t kTok = Dec::kTok;
   const uint32_t kvh = item.kvh, part = item.part, seq = item.seq, len = item.len;
   const uint32_t p0 = part * a.partition_tokens;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2543,7 +2716,6 @@ __device__ __forceinline__ void stream_item_shared(const DecodeArgs& a, uint8_t*
   dec.kbase = reinterpret_cast<uint64_t>(a.key_cache) + static_cast<uint64_t>(kvh) * a.k_head * es;
   dec.vbase = reinterpret_cast<uint64_t>(a.value_cache) + static_cast<uint64_t>(kvh) * a.v_head * es;
   dec.init_offsets();
-  uint8_t* vconv = tiles + S * Dec::kStageBytes + wave * (kStep * Dec::kPitch);  // FP8: this wave's 16-bit V
 
   float k_scale = 1.0f, v_scale = 1.0f;
   if (kFp8) {
@@ -2559,24 +2731,25 @@ __device__ __forceinline__ void stream_item_shared(const DecodeArgs& a, uint8_t*
     for (int dt = 0; dt < Dec::kDt; ++dt) dec.acc[ht][dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   }
 
-  const uint32_t nst = (dec.p1 - p0 + kStep - 1) / kStep;  // >= 1: the item holds tokens
-  const uint32_t t_last = p0 + (nst - 1) * kStep;
+  const uint32_t nst = (dec.p1 - p0 + kTok - 1) / kTok;  // >= 1: the item holds tokens
+  const uint32_t t_last = p0 + (nst - 1) * kTok;
+  if constexpr (kFp8) dec.odd = t_last + kStep >= dec.p1 ? 1U : 0U;
   // nx[j]: block of the next step that wave 0 loads into stage j (table
   // reads past the item's last step are clamped onto it; no K/V load is
   // issued past it).
-  uint32_t nx[S];
+  typename Dec::Blocks nx[S];
   if (wave == 0) {
-    uint32_t bk[S - 1];
+    typename Dec::Blocks bk[S - 1];
 #pragma unroll
-    for (int i = 0; i < S - 1; ++i) bk[i] = dec.block_of(min(p0 + i * kStep, t_last));
+    for (int i = 0; i < S - 1; ++i) bk[i] = dec.blocks_of(min(p0 + i * kTok, t_last));
 #pragma unroll
-    for (int i = 0; i < S - 1; ++i) nx[i] = dec.block_of(min(p0 + (S + i) * kStep, t_last));
-    nx[S - 1] = dec.block_of(min(p0 + (S - 1) * kStep, t_last));
+    for (int i = 0; i < S - 1; ++i) nx[i] = dec.blocks_of(min(p0 + (S + i) * kTok, t_last));
+    nx[S - 1] = dec.blocks_of(min(p0 + (S - 1) * kTok, t_last));
 #pragma unroll
-    for (int i = 0; i < S - 1; ++i) scalar_ready(bk[i]);
+    for (int i = 0; i < S - 1; ++i) bk[i].ready();
 #pragma unroll
     for (int i = 0; i < S - 1; ++i) {
-      if (i < nst) dec.issue(tiles + i * Dec::kStageBytes, bk[i], p0 + i * kStep);
+      if (i < nst) dec.issue(tiles + i * Dec::kStageBytes, bk[i], p0 + i * kTok);
     }
   }
   dec.load_query(seq, kvh * a.group + h0, a.group - h0);
@@ -2587,28 +2760,21 @@ __device__ __forceinline__ void stream_item_shared(const DecodeArgs& a, uint8_t*
 #pragma unroll
     for (int i = 0; i < S; ++i) {
       if (n + i < nst) {
-        const uint32_t t0 = p0 + (n + i) * kStep;
+        const uint32_t t0 = p0 + (n + i) * kTok;
         uint8_t* stage = tiles + i * Dec::kStageBytes;
         const int j = (i + S - 1) % S;  // the stage of the previous step
         if (wave == 0) {
           // this step's loads; the later steps' (up to S - 2) stay in flight
-          LOOM_WAVE_STALL(n + i, nst, (vm_wait_dma_later<Dec::kDmaPerStep, S - 2>(nst - 1 - (n + i))));
-          if (!kFp8) dec.zero_dead_rows(stage + Dec::kVOff, t0);
+          LOOM_WAVE_STALL(n + i, nst, (dec.template wait_step<S - 2>(nst - 1 - (n + i))));
+          dec.zero_dead_rows(stage, t0);
         }
         lds_barrier();  // this step's stage is in LDS; every wave is done with the previous one
         if (wave == 0) {
-          scalar_ready(nx[j]);
-          if (n + i + S - 1 < nst) dec.issue(tiles + j * Dec::kStageBytes, nx[j], t0 + (S - 1) * kStep);
-          nx[j] = dec.block_of(min(t0 + (2 * S - 1) * kStep, t_last));
+          nx[j].ready();
+          if (n + i + S - 1 < nst) dec.issue(tiles + j * Dec::kStageBytes, nx[j], t0 + (S - 1) * kTok);
+          nx[j] = dec.blocks_of(min(t0 + (2 * S - 1) * kTok, t_last));
         }
-        uint8_t* vtile = kFp8 ? vconv : stage + Dec::kVOff;
-        if (kFp8) {
-          dec.stage_v_fp8(stage, vtile, t0);
-          wave_fence_lds();
-        }
-        f32x4 sc[kHTW];
-        dec.qk(stage, sc);
-        dec.softmax_pv(sc, t0, vtile);
+        dec.consume(stage, t0);
       }
     }
   }
@@ -2664,7 +2830,7 @@ __device__ __forceinline__ WorkItem direct_item(const DecodeArgs& a, uint32_t bi
 template <typename QE, bool kFp8, int kSplit, int kHT = 1, uint32_t kD = kDim, int kNt = -1>
 __global__ __launch_bounds__(kSplit * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void decode_stream_kernel(DecodeArgs a) {
-  constexpr int kS = kFp8 ? kStreamStagesFp8 : kStreamStages;
+  constexpr int kS = kStreamStages;
   using Dec = Decoder<QE, kFp8, kHT, kD, kS, kNt>;
   __shared__ __attribute__((aligned(16))) uint8_t tiles[kSplit * Dec::kWaveBytes];
   LOOM_WAVE_STAMP(blockIdx.x * kSplit + (threadIdx.x >> 6));
@@ -2683,17 +2849,13 @@ void decode_stream_kernel(DecodeArgs a) {
 constexpr int kStreamGroup = 4;
 // Pipeline stages of the grouped kernel's 16-bit waves.
 constexpr int kStreamGroupStages = 2;
-// FP8 caches (rows half as long, stages half as large): eight items per
-// workgroup, which covers all heads of a token row or block when Hkv = 8.
-// Measured against four: C4 210 -> 205.6 us, head size 64 112.6 -> 108.5,
-// 96 169.7 -> 164.4, 112 104.8 -> 98.6; 16-bit caches measured 1% slower
-// with eight (head size 64) and 6% slower at head size 128 (one workgroup of
-// 128 KiB per CU). With non-temporal K/V loads and partial stores, four
-// against eight: C4 decode 189.4-189.9 against 189.6-190.1 us (the same);
-// head size 96 82.9-84.2 against 79.9-80.3, 112 89.7-90.2 against 84.9-85.3
-// (eight faster). Head size 128 with more than two partitions takes four-item
-// workgroups that fold pairs of partitions instead (pair_eligible).
-constexpr int kStreamGroupFp8 = 8;
+// The same for FP8 caches: 32-token stages hold the bytes of a 16-bit cache's
+// 16-token ones. Eight items per workgroup leave one workgroup per CU at head
+// sizes 80-112 (call us, eight -> four, B=64, Hq 32 / Hkv 8, NHD and HND: 64
+// 94.1 -> 92.4 and 83.4 -> 77.3, 80 106.2 -> 102.3 and 88.2 -> 79.3, 96 106.1 ->
+// 95.4 and 92.7 -> 81.6, 112 95.6 -> 93.3 and 79.0 -> 79.0); two items lose the
+// adjacent heads (96 101.8, 80 122.7). Head size 128 with more than two
+// partitions folds pairs of partitions instead (pair_eligible).
 
 // kDirect: items in index order (KV head fastest, then partition, then
 // sequence) instead of the longest-first schedule, for the library's own
@@ -2738,7 +2900,7 @@ template <typename QE, bool kFp8, int kGroup, uint32_t kD = kDim, int kNt = -1, 
           bool kPair = false>
 __global__ __launch_bounds__(kGroup * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void decode_stream_group_kernel(DecodeArgs a) {
-  constexpr int kGroupStages = kFp8 ? kStreamStagesFp8 : kStreamGroupStages;
+  constexpr int kGroupStages = kStreamGroupStages;
   using Dec = Decoder<QE, kFp8, 1, kD, kGroupStages, kNt>;
   __shared__ __attribute__((aligned(16))) uint8_t tiles[kGroup * Dec::kWaveBytes];
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2787,9 +2949,8 @@ void decode_stream_group_kernel(DecodeArgs a) {
 template <typename QE, bool kFp8, int kWaves, uint32_t kD = kDim, int kHTW = 2>
 __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void decode_stream_heads_kernel(DecodeArgs a) {
-  using Dec = StreamDecoder<QE, kFp8, kHTW, kD>;
-  __shared__ __attribute__((aligned(16)))
-  uint8_t tiles[kSharedStages * Dec::kStageBytes + (kFp8 ? kWaves * kStep * Dec::kPitch : 0)];
+  using Dec = Decoder<QE, kFp8, kHTW, kD, kFp8 ? kSharedStagesFp8 : kSharedStages, -1>;
+  __shared__ __attribute__((aligned(16))) uint8_t tiles[Dec::kWaveBytes];
   rise_priority_with_dispatch<kFp8 && kHTW == 2>();
   LOOM_WAVE_STAMP(blockIdx.x * kWaves + (threadIdx.x >> 6));
   const WorkItem item = schedule_item(a, blockIdx.x);
@@ -3390,7 +3551,7 @@ int launch_stream(const DecodeArgs& args, uint64_t grid, hipStream_t stream) {
 template <typename QE, bool kFp8, uint32_t kD, int kNt = -1>
 int launch_stream_rot_nt(const DecodeArgs& args, uint64_t grid, uint32_t steps, hipStream_t stream) {
   if (grid >= 4096 || (grid >= 1024 && steps >= 8))
-    return launch_stream_group<QE, kFp8, kD, kFp8 ? kStreamGroupFp8 : kStreamGroup, kNt>(args, grid, stream);
+    return launch_stream_group<QE, kFp8, kD, kStreamGroup, kNt>(args, grid, stream);
   if (steps < 8) return launch_stream<QE, kFp8, 1, 1, kD, kNt>(args, grid, stream);
   return launch_stream<QE, kFp8, 4, 1, kD, kNt>(args, grid, stream);
 }
@@ -3468,9 +3629,7 @@ bool heads_stream_eligible(const Problem& p, uint64_t parts) {
 
 template <typename QE, bool kFp8, uint32_t kD>
 int launch_stream_heads(const DecodeArgs& args, uint64_t items, uint32_t group, hipStream_t stream) {
-  using Dec = StreamDecoder<QE, kFp8, 2, kD>;
   TimedLaunch timed(LOOM_HIP_KERNEL_DECODE, stream);
-  static_assert(4 * Dec::kWaveBytes <= 64 * 1024, "four waves' stages fit in 64 KiB of LDS");
   const dim3 grid(static_cast<uint32_t>(items));
   g_launch_kernel = "decode_stream_heads_kernel";
   // One head tile per wave for 16-bit caches up to 64 heads (BF16 PV splits
@@ -3762,8 +3921,8 @@ int run_typed(const Problem& p, hipStream_t stream) {
         status = fp8 ? launch_stream_heads2<QE, true, 64>(args, grid, stream)
                      : launch_stream_heads2<QE, false, 64>(args, grid, stream);
       } else if (grid >= 4096 || (grid >= 1024 && steps >= 8)) {
-        status = fp8 ? (dense_rows ? launch_stream_group<QE, true, 64, kStreamGroupFp8, 1>(args, grid, stream)
-                                   : launch_stream_group<QE, true, 64, kStreamGroupFp8>(args, grid, stream))
+        status = fp8 ? (dense_rows ? launch_stream_group<QE, true, 64, kStreamGroup, 1>(args, grid, stream)
+                                   : launch_stream_group<QE, true, 64>(args, grid, stream))
                      : launch_stream_group<QE, false, 64>(args, grid, stream);
       } else if (steps < 8) {
         status = fp8 ? (dense_rows ? launch_stream<QE, true, 1, 1, 64, 1>(args, grid, stream)
@@ -3799,9 +3958,7 @@ int run_typed(const Problem& p, hipStream_t stream) {
         // The library's own split runs its items in index order with each
         // item's first block IDs loaded alongside its length (C2 decode
         // 18.3-18.5 -> 17.5-17.7 us).
-        status = fp8 && pair_eligible(args, 4, true)
-                                      ? launch_stream_group<QE, true, kDim, 4>(args, grid, stream)
-                 : fp8                ? launch_stream_group<QE, true, kDim, kStreamGroupFp8>(args, grid, stream)
+        status = fp8                 ? launch_stream_group<QE, true>(args, grid, stream)
                  : p.direct_schedule ? launch_stream_group<QE, false, kDim, kStreamGroup, -1, true>(args, grid, stream)
                                      : launch_stream_group<QE, false>(args, grid, stream);
       } else if (steps < 8) {
