@@ -8,6 +8,8 @@ load, every call raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
@@ -158,6 +160,37 @@ def lib() -> ctypes.CDLL:
                 fn.restype = restype
             _lib = handle
     return _lib
+
+
+_calls = None
+_CALL_ENTRY_POINTS = (
+    "loom_hip_paged_decode_attention_extended_f32",
+    "loom_hip_paged_decode_attention_extended_f16",
+    "loom_hip_paged_decode_attention_extended_bf16",
+    "loom_hip_paged_decode_attention_extended_workspace_elements",
+    "loom_hip_views_paged_decode_workspace_elements",
+    "loom_hip_views_paged_decode_attention",
+    "loom_hip_views_rope_paged_kv_write",
+)
+
+
+def calls():
+    """The native call module (csrc/host_calls.cpp), bound to the loaded library's entry points."""
+    global _calls
+    if _calls is None:
+        handle = lib()
+        with _lock:
+            if _calls is None:
+                path = _build.CALLS_PATH
+                if not os.path.exists(path):
+                    raise ImportError(f"loom-hip call module not found at {path}; run `python -m attnarc_amd.build`")
+                loader = importlib.machinery.ExtensionFileLoader("_loom_hip_calls", path)
+                spec = importlib.util.spec_from_file_location("_loom_hip_calls", path, loader=loader)
+                module = importlib.util.module_from_spec(spec)
+                loader.exec_module(module)
+                module.bind(*(ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in _CALL_ENTRY_POINTS))
+                _calls = module
+    return _calls
 
 
 def status_string(status: int) -> str:

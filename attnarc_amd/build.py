@@ -96,6 +96,35 @@ def _compile_adapter(verbose: bool) -> None:
     os.replace(tmp, ADAPTER_LIB_PATH)
 
 
+CALLS_SOURCE = os.path.join(PKG_DIR, "csrc", "host_calls.cpp")
+CALLS_PATH = os.path.join(PKG_DIR, "_build", "_loom_hip_calls.so")
+
+
+def _compile_calls(verbose: bool) -> None:
+    """Host-only Python module of the operator calls (``attnarc_amd.ops``), for this interpreter and torch build."""
+    import sysconfig
+
+    import torch
+    import torch.utils.cpp_extension as ext
+
+    torch_lib = ext.library_paths()[0]
+    tmp = CALLS_PATH + ".tmp"
+    cmd = [
+        os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-DUSE_ROCM",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        f"-I{sysconfig.get_paths()['include']}",
+        *[f"-I{p}" for p in ext.include_paths()],
+        f"-I{os.path.join(REPO_DIR, 'include')}",
+        CALLS_SOURCE,
+        f"-L{torch_lib}", "-ltorch_python", "-ltorch_hip", "-ltorch_cpu", "-lc10", f"-Wl,-rpath,{torch_lib}",
+        "-o", tmp,
+    ]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.run(cmd, check=True)
+    os.replace(tmp, CALLS_PATH)
+
+
 WAVE_TRACE_LIB_PATH = os.path.join(PKG_DIR, "_build", "libloom_hip_wave_trace.so")
 
 
@@ -116,10 +145,12 @@ def build_wave_trace(verbose: bool = False) -> str:
 
 
 def build(verbose: bool = False, incremental: bool = False) -> str:
-    """Compile the kernel library, the HBM probe library and the torch adapter; returns the first's path."""
+    """Compile the kernel library, the HBM probe library, the torch adapter and the Python call module; returns
+    the first's path."""
     _compile(SOURCES, LIB_PATH, verbose, incremental)
     _compile([PROBE_SOURCE], PROBE_LIB_PATH, verbose, incremental)
     _compile_adapter(verbose)
+    _compile_calls(verbose)
     return LIB_PATH
 
 

@@ -6,7 +6,9 @@ argument meaning, default scale ``head_size ** -0.5`` and RuntimeError /
 ValueError behaviour. The tensor contract of the reference's adapter
 (python/csrc/attention.cpp:5-88) is not restated here: the operands go to the
 library as tensor views and its contract tables decide (include/
-loom_hip_views.h), the same code the torch Stable-ABI adapter uses.
+loom_hip_views.h), the same code the torch Stable-ABI adapter uses. Calls whose
+operands are ordinary GPU tensors go through the native call module
+(csrc/host_calls.cpp); the code here takes every other call and words refusals.
 Differences: no 1024-token context cap, and an extended entry point for FP8
 E4M3 caches, HND layouts, log-sum-exp output and fixed split-K partitions.
 
@@ -37,8 +39,9 @@ _FP8_DTYPES = tuple(
 
 
 def _require_inference_tensors(*tensors: torch.Tensor) -> None:
-    if any(t is not None and t.requires_grad for t in tensors):
-        raise ValueError("Loom Kernels operators are inference-only")
+    for t in tensors:
+        if t is not None and t.requires_grad:
+            raise ValueError("Loom Kernels operators are inference-only")
 
 
 _VIEW_DTYPES = {
@@ -150,6 +153,12 @@ def paged_decode_attention_out(
     _require_inference_tensors(query, key_cache, value_cache, output)
     if scale is None:
         scale = query.shape[-1] ** -0.5
+    if query.is_cuda:
+        status = _native.calls().decode_views(query, key_cache, value_cache, block_tables, sequence_lengths, output,
+                                              max_sequence_length, scale)
+        if status is not None:
+            _raise_unless_ok(status, "paged decode attention")
+            return output
     lib = _native.lib()
     views = _views(query, key_cache, value_cache, block_tables, sequence_lengths, output)
     max_sequence_length = int(max_sequence_length)
@@ -261,6 +270,14 @@ def paged_decode_attention_extended(
     (``output`` and ``lse`` must then be given when they are wanted, and no
     ``workspace`` is taken). Returns ``output`` or ``(output, lse)``.
     """
+    if query.is_cuda and not no_alloc:
+        done = _native.calls().decode_extended(
+            query, key_cache, value_cache, block_tables, sequence_lengths, max_sequence_length, scale, layout,
+            key_scales, value_scales, partition_tokens, output, lse, return_lse, workspace)
+        if type(done) is int:
+            _native.check(done, "Loom paged decode attention")
+        if done is not None:
+            return done
     _require_inference_tensors(query, key_cache, value_cache)
     if query.dim() != 3 or not query.is_contiguous():
         raise RuntimeError("Loom paged decode query must be a contiguous rank-3 tensor")
@@ -390,6 +407,12 @@ def rope_paged_kv_write_(
     checks the views and submits through the checked bridge. Returns
     ``(query, key, kv_cache)``.
     """
+    if query.is_cuda:
+        status = _native.calls().rope_write(query, key, value, positions, cos_sin_cache, kv_cache, key_scales,
+                                            value_scales, slot_mapping, is_neox)
+        if status is not None:
+            _raise_unless_ok(status, "RoPE+paged-KV")
+            return query, key, kv_cache
     _require_inference_tensors(query, key, value, cos_sin_cache, kv_cache, key_scales, value_scales)
     views = _views(query, key, value, positions, cos_sin_cache, kv_cache, key_scales, value_scales, slot_mapping)
     lib = _native.lib()

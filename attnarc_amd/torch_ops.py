@@ -136,10 +136,18 @@ def paged_decode_attention(
     """Paged MQA/GQA decode for one query token per sequence (ops/attention.py:126-154)."""
     if query.dim() != 3 or value_cache.dim() != 4:
         raise ValueError("paged decode query/value cache must have ranks 3 and 4")
-    output = torch.empty((query.shape[0], query.shape[1], value_cache.shape[3]), device=query.device,
-                         dtype=query.dtype)
-    return paged_decode_attention_out(query, key_cache, value_cache, block_tables, sequence_lengths, output,
-                                      max_sequence_length=max_sequence_length, scale=scale)
+    sequences, query_heads, head_size = query.shape
+    value_head_size = value_cache.shape[3]
+    if head_size == value_head_size:
+        output = torch.empty_like(query)  # half the host time of a sized allocation
+    else:
+        output = torch.empty((sequences, query_heads, value_head_size), device=query.device, dtype=query.dtype)
+    _ops._require_inference_tensors(query, key_cache, value_cache)
+    if scale is None:
+        scale = head_size ** -0.5
+    _paged_decode_attention(query, key_cache, value_cache, block_tables, sequence_lengths, output,
+                            int(max_sequence_length), float(scale))
+    return output
 
 
 def rope_paged_kv_write_(
