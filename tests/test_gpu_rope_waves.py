@@ -1,0 +1,65 @@
+"""The vector RoPE + paged K/V write at the edges of its waves of 64 chunks.
+
+Bit-exact, as the other tests of the write: against the CPU oracle where a
+token's chunks end inside a wave, fill it, or divide by one; and, for calls
+large enough to take the non-temporal hint, against the same tokens in small
+calls.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from attnarc_amd import ops
+from test_gpu_rope import check_case, cos_sin_cache, packed_cache
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("is_neox", [True, False])
+@pytest.mark.parametrize("encoding", ["native", "per-head"])
+@pytest.mark.parametrize("heads,head_size,rotary", [
+    ((5, 3), 80, 80),     # 70 chunks of BF16: a wave and six lanes
+    ((1, 1), 64, 16),     # one rotary chunk a head; 16 chunks a token
+    ((4, 4), 64, 32),     # exactly one wave of BF16 chunks (interleaved)
+    ((33, 1), 128, 128),
+    ((2, 2), 256, 64),    # long unrotated tails
+])
+def test_chunks_of_a_token(dtype, is_neox, encoding, heads, head_size, rotary):
+    for tokens in (1, 7):
+        check_case(dtype, "HND", encoding, is_neox, T=tokens, Hq=heads[0], Hkv=heads[1], D=head_size, rd=rotary,
+                   maxpos=64, NB=4, bs=4, seed=31)
+
+
+@pytest.mark.parametrize("dtype,cache,tokens,is_neox", [
+    (torch.bfloat16, torch.bfloat16, 8201, True), (torch.float16, torch.uint8, 9001, True),
+    (torch.bfloat16, torch.uint8, 9001, False), (torch.float32, torch.float32, 4203, False)])
+def test_large_calls_equal_small_ones(dtype, cache, tokens, is_neox):
+    # over 192 MiB of rows and cache as one call, a few MiB in pieces of 501 tokens
+    hq, hkv, d, bs = 32, 8, 128, 16
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    packed = torch.randn((tokens, (hq + 2 * hkv) * d), generator=gen, device=DEV).to(dtype)
+    pos = torch.randint(0, 512, (tokens,), generator=gen, device=DEV)
+    pos[5] = 600  # outside the table: left untouched
+    blocks = tokens // bs + 2
+    slots = torch.randperm(blocks * bs, generator=gen, device=DEV)[:tokens].contiguous()
+    slots[7] = -1
+    cs = cos_sin_cache(512, d, dtype)
+    ks, vs = (torch.rand(hkv, generator=gen, device=DEV) * 0.1 + 0.01 for _ in range(2))
+
+    def write(pieces):
+        rows = packed.clone()
+        kv = packed_cache(blocks, bs, hkv, d, cache, "HND")
+        q, k, v = (x.unflatten(1, (-1, d)) for x in rows.split((hq * d, hkv * d, hkv * d), dim=1))
+        for part in torch.arange(tokens, device=DEV).split(tokens if pieces == 1 else 501):
+            a, b = int(part[0]), int(part[-1]) + 1
+            ops.rope_paged_kv_write_(q[a:b], k[a:b], v[a:b], pos[a:b].contiguous(), cs, kv, ks, vs,
+                                     slots[a:b].contiguous(), is_neox)
+        torch.cuda.synchronize()
+        return rows, kv
+
+    (rows, kv), (want_rows, want_kv) = write(1), write(0)
+    assert torch.equal(rows, want_rows) and torch.equal(kv, want_kv)
