@@ -2683,21 +2683,25 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 constexpr int kSharedStages = 4;
 constexpr int kSharedStagesFp8 = 3;
 
-// One work item of a group of 33-128 query heads: kWaves waves, wave w
-// computing heads 32 w .. 32 w + 31 with two head tiles, from a ring of K/V
-// stages that all waves share. Wave 0 issues every step's DMA. One barrier
-// per step, after wave 0's wait for the step's stage, both publishes that
-// stage and shows that every wave has finished the previous step, whose
-// stage wave 0 then refills (S - 1 steps ahead). The waves have the same
-// steps, so all of them reach every barrier.
-template <typename QE, bool kFp8, int kWaves, uint32_t kD, int kHTW = 2>
-__device__ __forceinline__ void stream_item_shared(const DecodeArgs& a, uint8_t* tiles, const WorkItem& item) {
+// One work item of a wide group of query heads: kRings rings of K/V stages,
+// each read by kWaves waves, wave w of a ring computing kHTW head tiles from
+// head 16 kHTW w on. Ring r takes the item's steps r, r + kRings, ...; its wave
+// 0 issues every step's DMA. One barrier per step, after wave 0's wait for the
+// step's stage, both publishes that stage and shows that every wave has
+// finished the previous step, whose stage wave 0 then refills (S - 1 steps
+// ahead). All waves reach every barrier: a ring without a last step only waits
+// there. The rings' states are combined in LDS at the end.
+template <typename QE, bool kFp8, int kWaves, uint32_t kD, int kHTW = 2, int kRings = 1>
+__device__ __forceinline__ void stream_item_shared(const DecodeArgs& a, uint8_t* lds, const WorkItem& item) {
   constexpr int S = kFp8 ? kSharedStagesFp8 : kSharedStages;
   using Dec = Decoder<QE, kFp8, kHTW, kD, S, -1>;
   constexpr uint32_t kTok = Dec::kTok;
   const uint32_t kvh = item.kvh, part = item.part, seq = item.seq, len = item.len;
   const uint32_t p0 = part * a.partition_tokens;
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t wg_wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t ring = kRings == 1 ? 0U : wg_wave / kWaves;
+  const uint32_t wave = kRings == 1 ? wg_wave : wg_wave % kWaves;
+  uint8_t* tiles = lds + ring * Dec::kWaveBytes;
   const uint32_t h0 = wave * 16U * kHTW;
 
   Dec dec(a);
@@ -2731,50 +2735,57 @@ __device__ __forceinline__ void stream_item_shared(const DecodeArgs& a, uint8_t*
     for (int dt = 0; dt < Dec::kDt; ++dt) dec.acc[ht][dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   }
 
-  const uint32_t nst = (dec.p1 - p0 + kTok - 1) / kTok;  // >= 1: the item holds tokens
-  const uint32_t t_last = p0 + (nst - 1) * kTok;
+  const uint32_t steps = (dec.p1 - p0 + kTok - 1) / kTok;  // >= 1: the item holds tokens
+  const uint32_t nst = steps > ring ? (steps - ring + kRings - 1) / kRings : 0U;  // this ring's
+  const uint32_t rounds = (steps + kRings - 1) / kRings;                          // ring 0's: the most
+  constexpr uint32_t st = kRings * kTok;
+  const uint32_t t_first = p0 + ring * kTok;
+  const uint32_t t_last = t_first + (nst > 0 ? nst - 1 : 0U) * st;
   if constexpr (kFp8) dec.odd = t_last + kStep >= dec.p1 ? 1U : 0U;
   // nx[j]: block of the next step that wave 0 loads into stage j (table
   // reads past the item's last step are clamped onto it; no K/V load is
   // issued past it).
   typename Dec::Blocks nx[S];
-  if (wave == 0) {
+  if (wave == 0 && nst > 0) {
     typename Dec::Blocks bk[S - 1];
 #pragma unroll
-    for (int i = 0; i < S - 1; ++i) bk[i] = dec.blocks_of(min(p0 + i * kTok, t_last));
+    for (int i = 0; i < S - 1; ++i) bk[i] = dec.blocks_of(min(t_first + i * st, t_last));
 #pragma unroll
-    for (int i = 0; i < S - 1; ++i) nx[i] = dec.blocks_of(min(p0 + (S + i) * kTok, t_last));
-    nx[S - 1] = dec.blocks_of(min(p0 + (S - 1) * kTok, t_last));
+    for (int i = 0; i < S - 1; ++i) nx[i] = dec.blocks_of(min(t_first + (S + i) * st, t_last));
+    nx[S - 1] = dec.blocks_of(min(t_first + (S - 1) * st, t_last));
 #pragma unroll
     for (int i = 0; i < S - 1; ++i) bk[i].ready();
 #pragma unroll
     for (int i = 0; i < S - 1; ++i) {
-      if (i < nst) dec.issue(tiles + i * Dec::kStageBytes, bk[i], p0 + i * kTok);
+      if (i < nst) dec.issue(tiles + i * Dec::kStageBytes, bk[i], t_first + i * st);
     }
   }
   dec.load_query(seq, kvh * a.group + h0, a.group - h0);
 
   LOOM_WAVE_STALL_DECL;
-  for (uint32_t n = 0; n < nst; n += S) {
+  for (uint32_t n = 0; n < rounds; n += S) {
     if (wave == 0) LOOM_WAVE_MARK(n, S, nst);
 #pragma unroll
     for (int i = 0; i < S; ++i) {
-      if (n + i < nst) {
-        const uint32_t t0 = p0 + (n + i) * kTok;
+      if (n + i < rounds) {
+        const bool mine = kRings == 1 || n + i < nst;  // uniform per wave; false only in the last round
+        const uint32_t t0 = t_first + (n + i) * st;
         uint8_t* stage = tiles + i * Dec::kStageBytes;
         const int j = (i + S - 1) % S;  // the stage of the previous step
-        if (wave == 0) {
+        if (wave == 0 && mine) {
           // this step's loads; the later steps' (up to S - 2) stay in flight
           LOOM_WAVE_STALL(n + i, nst, (dec.template wait_step<S - 2>(nst - 1 - (n + i))));
           dec.zero_dead_rows(stage, t0);
         }
         lds_barrier();  // this step's stage is in LDS; every wave is done with the previous one
-        if (wave == 0) {
-          nx[j].ready();
-          if (n + i + S - 1 < nst) dec.issue(tiles + j * Dec::kStageBytes, nx[j], t0 + (S - 1) * kTok);
-          nx[j] = dec.blocks_of(min(t0 + (2 * S - 1) * kTok, t_last));
+        if (mine) {
+          if (wave == 0) {
+            nx[j].ready();
+            if (n + i + S - 1 < nst) dec.issue(tiles + j * Dec::kStageBytes, nx[j], t0 + (S - 1) * st);
+            nx[j] = dec.blocks_of(min(t0 + (2 * S - 1) * st, t_last));
+          }
+          dec.consume(stage, t0);
         }
-        dec.consume(stage, t0);
       }
     }
   }
@@ -2785,7 +2796,19 @@ __device__ __forceinline__ void stream_item_shared(const DecodeArgs& a, uint8_t*
 
 #pragma unroll
   for (int ht = 0; ht < kHTW; ++ht) {
-    const float l = head_sum(dec.lsum[ht]);
+    float l = head_sum(dec.lsum[ht]);
+    if constexpr (kRings > 1) {
+      // Rings 1 .. hand tile ht's state to ring 0's wave of the same heads.
+      constexpr uint32_t kStateBytes = Dec::kDt * 1024 + 512;
+      static_assert((kRings - 1) * kWaves * kStateBytes <= kRings * Dec::kWaveBytes, "the states fit the stages");
+      __syncthreads();  // every wave is done with the stages, or with the previous tile's states
+      if (ring > 0) pair_publish<Dec>(lds + ((ring - 1) * kWaves + wave) * kStateBytes, dec.m[ht], l, dec.acc[ht]);
+      __syncthreads();
+      if (ring > 0) continue;
+#pragma unroll
+      for (int o = 0; o < kRings - 1; ++o)
+        pair_combine<Dec>(lds + (o * kWaves + wave) * kStateBytes, dec.m[ht], l, dec.acc[ht]);
+    }
     if (h0 + ht * 16U + dec.c < a.group)
       store_wave_result<QE>(a, dec, ht, seq, kvh * a.group + h0 + ht * 16U, part, v_scale, l);
   }
@@ -2946,17 +2969,17 @@ void decode_stream_group_kernel(DecodeArgs a) {
 // Groups of 17-128 query heads: one workgroup of waves of 16 or 32 heads each
 // (kHTW head tiles of 16) per work item (stream_item_shared), so that each K/V
 // row is read from HBM once into LDS for all of the group's heads.
-template <typename QE, bool kFp8, int kWaves, uint32_t kD = kDim, int kHTW = 2>
-__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
+template <typename QE, bool kFp8, int kWaves, uint32_t kD = kDim, int kHTW = 2, int kRings = 1>
+__global__ __launch_bounds__(kRings * kWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void decode_stream_heads_kernel(DecodeArgs a) {
   using Dec = Decoder<QE, kFp8, kHTW, kD, kFp8 ? kSharedStagesFp8 : kSharedStages, -1>;
-  __shared__ __attribute__((aligned(16))) uint8_t tiles[Dec::kWaveBytes];
+  __shared__ __attribute__((aligned(16))) uint8_t tiles[kRings * Dec::kWaveBytes];
   rise_priority_with_dispatch<kFp8 && kHTW == 2>();
-  LOOM_WAVE_STAMP(blockIdx.x * kWaves + (threadIdx.x >> 6));
+  LOOM_WAVE_STAMP(blockIdx.x * kRings * kWaves + (threadIdx.x >> 6));
   const WorkItem item = schedule_item(a, blockIdx.x);
   if (threadIdx.x < 64) LOOM_WAVE_ITEM(a, item);  // one record per item: the waves share its K/V reads
   if (!item.valid) return;  // uniform across the workgroup
-  stream_item_shared<QE, kFp8, kWaves, kD, kHTW>(a, tiles, item);
+  stream_item_shared<QE, kFp8, kWaves, kD, kHTW, kRings>(a, tiles, item);
 }
 
 // ---------------------------------------------------------------------------
@@ -3627,58 +3650,74 @@ bool heads_stream_eligible(const Problem& p, uint64_t parts) {
          15 * p.k_page * es + 256 < limit && 15 * p.v_page * es + 256 < limit;
 }
 
+// Up to this many items every workgroup of a wide group has a CU to itself and
+// its time is one ring's latency per step: several rings share the item's
+// steps. Call us with 1 / 2 / 4 rings at 32, 256 and 384 items of 512 tokens: BF16
+// 32/1 28.4 / 22.7 / 18.9, 30.3 / 25.4 / 22.8, 32.6 / 28.9 / 38.4; FP8 32/1 23.0 /
+// 16.8 / 15.9, 24.9 / 19.1 / 18.5, 26.1 / 22.3 / 30.7; BF16 48/1 28.8 / 21.0 / 20.2,
+// 31.4 / 24.4 / 24.5, 33.7 / 41.0 / 41.7; FP8 64/1 28.6 / 20.1 / 20.8, 31.6 / 23.8 /
+// 25.0, 36.4 / 29.7 / 42.6; BF16 96/1 37.5 / 29.4 / -, 42.5 / 35.3 / -, 51.8 / 60.3 /
+// -; 160 tokens x 30 FP8 32/1 10.2 / 9.2 / 9.6.
+constexpr uint64_t kHeadsSmallGrid = 256;
+
+template <typename QE, bool kFp8, int kWaves, uint32_t kD, int kHTW, int kRings = 1>
+int launch_heads_kernel(const DecodeArgs& args, uint64_t items, hipStream_t stream) {
+  TimedLaunch timed(LOOM_HIP_KERNEL_DECODE, stream);
+  g_launch_kernel = "decode_stream_heads_kernel";
+  hipLaunchKernelGGL((decode_stream_heads_kernel<QE, kFp8, kWaves, kD, kHTW, kRings>),
+                     dim3(static_cast<uint32_t>(items)), dim3(kRings * kWaves * 64), 0, stream, args);
+  return hipGetLastError() == hipSuccess ? LOOM_HIP_SUCCESS : LOOM_HIP_LAUNCH_ERROR;
+}
+
 template <typename QE, bool kFp8, uint32_t kD>
 int launch_stream_heads(const DecodeArgs& args, uint64_t items, uint32_t group, hipStream_t stream) {
-  TimedLaunch timed(LOOM_HIP_KERNEL_DECODE, stream);
-  const dim3 grid(static_cast<uint32_t>(items));
-  g_launch_kernel = "decode_stream_heads_kernel";
+  const bool small = items <= kHeadsSmallGrid;
   // One head tile per wave for 16-bit caches up to 64 heads (BF16 PV splits
   // probabilities into hi + lo, two MFMAs per tile; F16 48/1 and 64/1 gain
   // 3.5 us as well), and for FP8 groups of up to 48 heads, whose second wave
   // would otherwise hold a half-empty tile. Decode us, two-tile waves ->
   // one-tile waves (B=64, 16384 tokens, 512-token partitions): BF16 48/1
-  // 120.4 -> 109.7, 64/1 124.5 -> 112.9, head size 64 48/1 62.2 -> 56.0;
-  // FP8 48/1 102.8 -> 98.3, FP8 64/1 105.6 -> 107.1 (kept on two tiles).
-  if ((!kFp8 && group <= 64) || group <= 48) {
-    if (group <= 48)
-      hipLaunchKernelGGL((decode_stream_heads_kernel<QE, kFp8, 3, kD, 1>), grid, dim3(192), 0, stream, args);
-    else
-      hipLaunchKernelGGL((decode_stream_heads_kernel<QE, kFp8, 4, kD, 1>), grid, dim3(256), 0, stream, args);
-    return hipGetLastError() == hipSuccess ? LOOM_HIP_SUCCESS : LOOM_HIP_LAUNCH_ERROR;
-  }
-  // 16-bit caches with groups of 97-128: seven or eight one-tile waves (BF16
-  // 128/1, 8192 tokens: 93.3 -> 88.4 us). Groups of 65-96 stay on three two-tile
-  // waves: six one-tile waves took 102 us against 70.
-  if (!kFp8 && group > 96) {
-    // ceil(group / 16) waves, so that every wave holds a live head
-    if (group <= 112)
-      hipLaunchKernelGGL((decode_stream_heads_kernel<QE, kFp8, 7, kD, 1>), grid, dim3(448), 0, stream, args);
-    else
-      hipLaunchKernelGGL((decode_stream_heads_kernel<QE, kFp8, 8, kD, 1>), grid, dim3(512), 0, stream, args);
-    return hipGetLastError() == hipSuccess ? LOOM_HIP_SUCCESS : LOOM_HIP_LAUNCH_ERROR;
-  }
+  // 120.4 -> 109.7, 64/1 124.5 -> 112.9, head size 64 48/1 62.2 -> 56.0. Call
+  // us, FP8 64/1 x 8192 45.9 -> 47.5 (kept on two tiles).
+  if (group <= 48)
+    return small ? launch_heads_kernel<QE, kFp8, 3, kD, 1, 2>(args, items, stream)
+                 : launch_heads_kernel<QE, kFp8, 3, kD, 1>(args, items, stream);
   if (group <= 64) {
-    hipLaunchKernelGGL((decode_stream_heads_kernel<QE, kFp8, 2, kD>), grid, dim3(128), 0, stream, args);
-  } else if (group <= 96) {
-    hipLaunchKernelGGL((decode_stream_heads_kernel<QE, kFp8, 3, kD>), grid, dim3(192), 0, stream, args);
-  } else {
-    hipLaunchKernelGGL((decode_stream_heads_kernel<QE, kFp8, 4, kD>), grid, dim3(256), 0, stream, args);
+    // FP8 keeps two rings to 512 items (384: 36.4 -> 29.7, 512: 38.1 -> 32.3)
+    if constexpr (kFp8)
+      return items <= 2 * kHeadsSmallGrid ? launch_heads_kernel<QE, kFp8, 2, kD, 2, 2>(args, items, stream)
+                                          : launch_heads_kernel<QE, kFp8, 2, kD, 2>(args, items, stream);
+    return small ? launch_heads_kernel<QE, kFp8, 4, kD, 1, 2>(args, items, stream)
+                 : launch_heads_kernel<QE, kFp8, 4, kD, 1>(args, items, stream);
   }
-  return hipGetLastError() == hipSuccess ? LOOM_HIP_SUCCESS : LOOM_HIP_LAUNCH_ERROR;
+  // Groups of 65-96 stay on three two-tile waves: six one-tile waves took 102
+  // us against 70 (FP8 71.3 against 60.4).
+  if (group <= 96)
+    return small ? launch_heads_kernel<QE, kFp8, 3, kD, 2, 2>(args, items, stream)
+                 : launch_heads_kernel<QE, kFp8, 3, kD, 2>(args, items, stream);
+  // Groups of 97-128: ceil(group / 16) one-tile waves, so that every wave holds
+  // a live head (BF16 128/1, 8192 tokens: 93.3 -> 88.4 us). FP8 only on small
+  // grids (2048 tokens: 32 items 29.8 -> 26.2, 256 34.3 -> 30.6; 384 46.4 ->
+  // 46.5, 64 x 8192 67.9 -> 78.4).
+  if (!kFp8 || small) {
+    if (group <= 112) return launch_heads_kernel<QE, kFp8, 7, kD, 1>(args, items, stream);
+    return launch_heads_kernel<QE, kFp8, 8, kD, 1>(args, items, stream);
+  }
+  return launch_heads_kernel<QE, kFp8, 4, kD, 2>(args, items, stream);
 }
 
-// Groups of 17-32 query heads as two waves of 16 heads on one shared ring of
-// K/V stages (decode_stream_heads_kernel with one head tile per wave). With
+// Groups of 17-32 query heads as two waves of 16 heads per ring of K/V stages
+// (decode_stream_heads_kernel with one head tile per wave). With
 // PV taking BF16 probabilities as hi + lo, a wave holding both head tiles
 // became bound by its own MFMA and softmax chain at ~3 waves per CU: C5
-// decode 74.7 us as one wave per item, 70.2 us as two.
+// decode 74.7 us as one wave per item, 70.2 us as two. Two rings to 512 items
+// (384 and 512: BF16 32.6 -> 28.9 and 34.1 -> 33.5, FP8 26.1 -> 22.3 and 27.3 ->
+// 23.7).
 template <typename QE, bool kFp8, uint32_t kD>
 int launch_stream_heads2(const DecodeArgs& args, uint64_t items, hipStream_t stream) {
-  TimedLaunch timed(LOOM_HIP_KERNEL_DECODE, stream);
-  g_launch_kernel = "decode_stream_heads_kernel";
-  hipLaunchKernelGGL((decode_stream_heads_kernel<QE, kFp8, 2, kD, 1>), dim3(static_cast<uint32_t>(items)), dim3(128), 0,
-                     stream, args);
-  return hipGetLastError() == hipSuccess ? LOOM_HIP_SUCCESS : LOOM_HIP_LAUNCH_ERROR;
+  if (items <= kHeadsSmallGrid) return launch_heads_kernel<QE, kFp8, 2, kD, 1, 4>(args, items, stream);
+  if (items <= 2 * kHeadsSmallGrid) return launch_heads_kernel<QE, kFp8, 2, kD, 1, 2>(args, items, stream);
+  return launch_heads_kernel<QE, kFp8, 2, kD, 1>(args, items, stream);
 }
 
 bool narrow_stream_eligible(const Problem& p, uint64_t parts, uint32_t group) {
