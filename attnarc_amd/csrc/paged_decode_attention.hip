@@ -1236,6 +1236,18 @@ struct StepBlocks {
 // stages than with 2).
 constexpr int kStreamStages = 2;
 
+// One stage per wave (the next step's loads go out when the step has been
+// consumed) holds as many bytes in flight per CU with twice the waves: finer
+// shares, and more waves to compute while others wait. It pays where the items
+// fill the waves. Call us, two stages -> one: head size 256, single waves, 64
+// x 2048 16-bit 180 -> 171, FP8 98.5 -> 91.9, 44 ragged sequences 111 -> 94.8 and
+// 74.8 -> 62.5; head size 128 16-bit (two-item workgroups) 64 x 512-8192 195.8 ->
+// 190.3, 44 x <= 2874 63.3 -> 52.4, 66 x <= 1015 44.5 -> 42.9, but 1,368 items
+// 43.6 -> 48.8; FP8 pairs 57 x <= 1998 38.1 -> 33.6, 128 x 4096 188.2 -> 187.9.
+// Head sizes 64-112 keep two (96 NHD ragged 169 -> 175, 64 57 x <= 3000 26.4 ->
+// 39.8).
+constexpr uint64_t kOneStageItems = 2048;
+
 // kHT: 16-query-head tiles per wave (1, or 2 for groups of 17-32 heads). The
 // tiles share each step's K operand fetches and V transposed reads.
 // kD: head size (= value head size): 128; 64, whose rows of 128 bytes come
@@ -1845,7 +1857,9 @@ struct Fp8StreamDecoder {
   static constexpr uint32_t kVOff1 = 3 * kHalfBytes + (kSwz ? 0U : kD == 96 ? 16U : 128U);
   static constexpr int kStages = kS;
   static constexpr uint32_t kStageBytes = kVOff1 + kHalfBytes;
-  static constexpr uint32_t kWaveBytes = kStages * kStageBytes;
+  // at least a published state (pair_publish)
+  static constexpr uint32_t kWaveBytes =
+      kStages * kStageBytes > kDt * 1024 + 512 ? kStages * kStageBytes : kDt * 1024 + 512;
   using Ops = MfmaOps<QE>;
   using vec8 = typename Ops::vec8;
   using PvOps = MfmaOps<F16Elem>;
@@ -2489,7 +2503,7 @@ __device__ __forceinline__ void stream_item(const DecodeArgs& a, uint8_t* tiles,
   const uint32_t seq = item.seq;
   const uint32_t len = item.len;
   const uint32_t p0 = part * a.partition_tokens;
-  static_assert(Dec::kWaveBytes >= 16 * (kD + 4) * sizeof(float),
+  static_assert(kSplit == 1 || Dec::kWaveBytes >= 16 * (kD + 4) * sizeof(float),
                 "the cross-wave reduction reuses the stages");
 
   Dec dec(a);
@@ -2850,10 +2864,9 @@ __device__ __forceinline__ WorkItem direct_item(const DecodeArgs& a, uint32_t bi
   return item;
 }
 
-template <typename QE, bool kFp8, int kSplit, int kHT = 1, uint32_t kD = kDim, int kNt = -1>
+template <typename QE, bool kFp8, int kSplit, int kHT = 1, uint32_t kD = kDim, int kNt = -1, int kS = kStreamStages>
 __global__ __launch_bounds__(kSplit * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void decode_stream_kernel(DecodeArgs a) {
-  constexpr int kS = kStreamStages;
   using Dec = Decoder<QE, kFp8, kHT, kD, kS, kNt>;
   __shared__ __attribute__((aligned(16))) uint8_t tiles[kSplit * Dec::kWaveBytes];
   LOOM_WAVE_STAMP(blockIdx.x * kSplit + (threadIdx.x >> 6));
@@ -2870,8 +2883,6 @@ void decode_stream_kernel(DecodeArgs a) {
 // requested from one CU at about the same time, which the memory system
 // serves faster than the same rows requested from CUs on different XCDs.
 constexpr int kStreamGroup = 4;
-// Pipeline stages of the grouped kernel's 16-bit waves.
-constexpr int kStreamGroupStages = 2;
 // The same for FP8 caches: 32-token stages hold the bytes of a 16-bit cache's
 // 16-token ones. Eight items per workgroup leave one workgroup per CU at head
 // sizes 80-112 (call us, eight -> four, B=64, Hq 32 / Hkv 8, NHD and HND: 64
@@ -2920,10 +2931,9 @@ __device__ __forceinline__ void rise_priority_with_dispatch() {
 }
 
 template <typename QE, bool kFp8, int kGroup, uint32_t kD = kDim, int kNt = -1, bool kDirect = false,
-          bool kPair = false>
+          bool kPair = false, int kGroupStages = kStreamStages>
 __global__ __launch_bounds__(kGroup * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void decode_stream_group_kernel(DecodeArgs a) {
-  constexpr int kGroupStages = kStreamGroupStages;
   using Dec = Decoder<QE, kFp8, 1, kD, kGroupStages, kNt>;
   __shared__ __attribute__((aligned(16))) uint8_t tiles[kGroup * Dec::kWaveBytes];
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -3535,7 +3545,8 @@ bool pair_eligible(const DecodeArgs& a, int group, bool fp8) {
   return fp8 && a.head_size == kDim && a.parts > 2 && group >= 4 && a.kv_heads % static_cast<uint32_t>(group / 2) == 0;
 }
 
-template <typename QE, bool kFp8, uint32_t kD = kDim, int kGroup = kStreamGroup, int kNt = -1, bool kDirect = false>
+template <typename QE, bool kFp8, uint32_t kD = kDim, int kGroup = kStreamGroup, int kNt = -1, bool kDirect = false,
+          int kS = kStreamStages>
 int launch_stream_group(const DecodeArgs& args, uint64_t items, hipStream_t stream) {
   TimedLaunch timed(LOOM_HIP_KERNEL_DECODE, stream);
   g_launch_kernel = "decode_stream_group_kernel";
@@ -3547,24 +3558,24 @@ int launch_stream_group(const DecodeArgs& args, uint64_t items, hipStream_t stre
     if (g_launch_pairs) {
       // one workgroup per (sequence, pair of partitions, group of kGroup / 2 KV heads)
       const uint64_t units = (args.parts + 1ULL) / 2ULL * args.sequences * (args.kv_heads / (kGroup / 2));
-      hipLaunchKernelGGL((decode_stream_group_kernel<QE, kFp8, kGroup, kD, kNt, false, true>),
+      hipLaunchKernelGGL((decode_stream_group_kernel<QE, kFp8, kGroup, kD, kNt, false, true, kS>),
                          dim3(static_cast<uint32_t>(units)), dim3(kGroup * 64), 0, stream, args);
       return hipGetLastError() == hipSuccess ? LOOM_HIP_SUCCESS : LOOM_HIP_LAUNCH_ERROR;
     }
   }
   {
     const uint64_t groups = (items + kGroup - 1) / kGroup;
-    hipLaunchKernelGGL((decode_stream_group_kernel<QE, kFp8, kGroup, kD, kNt, kDirect>),
+    hipLaunchKernelGGL((decode_stream_group_kernel<QE, kFp8, kGroup, kD, kNt, kDirect, false, kS>),
                        dim3(static_cast<uint32_t>(groups)), dim3(kGroup * 64), 0, stream, args);
   }
   return hipGetLastError() == hipSuccess ? LOOM_HIP_SUCCESS : LOOM_HIP_LAUNCH_ERROR;
 }
 
-template <typename QE, bool kFp8, int kSplit, int kHT = 1, uint32_t kD = kDim, int kNt = -1>
+template <typename QE, bool kFp8, int kSplit, int kHT = 1, uint32_t kD = kDim, int kNt = -1, int kS = kStreamStages>
 int launch_stream(const DecodeArgs& args, uint64_t grid, hipStream_t stream) {
   TimedLaunch timed(LOOM_HIP_KERNEL_DECODE, stream);
   g_launch_kernel = "decode_stream_kernel";
-  hipLaunchKernelGGL((decode_stream_kernel<QE, kFp8, kSplit, kHT, kD, kNt>), dim3(static_cast<uint32_t>(grid)),
+  hipLaunchKernelGGL((decode_stream_kernel<QE, kFp8, kSplit, kHT, kD, kNt, kS>), dim3(static_cast<uint32_t>(grid)),
                      dim3(kSplit * 64), 0, stream, args);
   return hipGetLastError() == hipSuccess ? LOOM_HIP_SUCCESS : LOOM_HIP_LAUNCH_ERROR;
 }
@@ -3942,14 +3953,18 @@ int run_typed(const Problem& p, hipStream_t stream) {
         status = fp8 ? launch_stream_rot<QE, true, 112>(args, grid, steps, dense_rows, stream)
                      : launch_stream_rot<QE, false, 112>(args, grid, steps, dense_rows, stream);
       } else if (p.head_size == 256) {
-        // 32 KiB of LDS per wave: two items per grouped workgroup, and the
-        // 4-wave split (129 KiB, one workgroup per CU) only for grids under
-        // 4 items per CU (measured: 1024-2048 items ran 11-15% faster as
-        // one wave per item; 128 items 1.6x slower).
+        // 16 KiB of LDS per stage: one stage per wave from 1024 items (two
+        // items per workgroup from 4096), and the 4-wave split (two stages,
+        // 129 KiB, one workgroup per CU) for grids under 4 items per CU
+        // (measured: 1024-2048 items ran 11-15% faster as one wave per item;
+        // 128 items 1.6x slower).
         if (grid >= 4096) {
-          status = fp8 ? launch_stream_group<QE, true, 256, 2>(args, grid, stream)
-                       : launch_stream_group<QE, false, 256, 2>(args, grid, stream);
-        } else if (grid >= 1024 || steps < 8) {
+          status = fp8 ? launch_stream_group<QE, true, 256, 2, -1, false, 1>(args, grid, stream)
+                       : launch_stream_group<QE, false, 256, 2, -1, false, 1>(args, grid, stream);
+        } else if (grid >= 1024) {
+          status = fp8 ? launch_stream<QE, true, 1, 1, 256, -1, 1>(args, grid, stream)
+                       : launch_stream<QE, false, 1, 1, 256, -1, 1>(args, grid, stream);
+        } else if (steps < 8) {
           status = fp8 ? launch_stream<QE, true, 1, 1, 256>(args, grid, stream)
                        : launch_stream<QE, false, 1, 1, 256>(args, grid, stream);
         } else {
@@ -3997,7 +4012,11 @@ int run_typed(const Problem& p, hipStream_t stream) {
         // The library's own split runs its items in index order with each
         // item's first block IDs loaded alongside its length (C2 decode
         // 18.3-18.5 -> 17.5-17.7 us).
-        status = fp8                 ? launch_stream_group<QE, true>(args, grid, stream)
+        const bool one_stage = grid >= kOneStageItems && steps >= 8;
+        status = fp8 ? (one_stage ? launch_stream_group<QE, true, kDim, kStreamGroup, -1, false, 1>(args, grid, stream)
+                                  : launch_stream_group<QE, true>(args, grid, stream))
+                 : one_stage && !p.direct_schedule
+                     ? launch_stream_group<QE, false, kDim, 2, -1, false, 1>(args, grid, stream)
                  : p.direct_schedule ? launch_stream_group<QE, false, kDim, kStreamGroup, -1, true>(args, grid, stream)
                                      : launch_stream_group<QE, false>(args, grid, stream);
       } else if (steps < 8) {
