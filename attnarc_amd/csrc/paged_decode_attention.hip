@@ -3542,7 +3542,13 @@ int launch_mfma_waves(const DecodeArgs& args, uint64_t grid, uint32_t chunks, hi
 // against 115.3, 80 134.2 against 132.7, 96 131.2 against 129.3, 112 105.5
 // against 104.4.
 bool pair_eligible(const DecodeArgs& a, int group, bool fp8) {
-  return fp8 && a.head_size == kDim && a.parts > 2 && group >= 4 && a.kv_heads % static_cast<uint32_t>(group / 2) == 0;
+  // The states are worth folding where a KV head has eight query heads, or four
+  // in an HND cache. Call us, pairs -> none: 16/8 x 1000-2000 x 100 NHD 72.3 ->
+  // 63.6, HND 68.3 -> 62.3, 24/4 NHD 57.6 -> 50.3, 32/32 x <= 1500 NHD 128.6 ->
+  // 125.2, 32/8 NHD 512-8192 111.1 -> 107.9; 32/8 HND 2000-4000 49.3 -> 52.5, 64/8
+  // 33.6 -> 36.7.
+  const bool folds = a.group >= 8 || (a.group >= 4 && a.k_page == a.head_size && a.v_page == a.head_size);
+  return folds && fp8 && a.head_size == kDim && a.parts > 2 && group >= 4 && a.kv_heads % static_cast<uint32_t>(group / 2) == 0;
 }
 
 template <typename QE, bool kFp8, uint32_t kD = kDim, int kGroup = kStreamGroup, int kNt = -1, bool kDirect = false,
@@ -3580,13 +3586,33 @@ int launch_stream(const DecodeArgs& args, uint64_t grid, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? LOOM_HIP_SUCCESS : LOOM_HIP_LAUNCH_ERROR;
 }
 
+// Items of fewer than eight 16-token steps on grids that leave CUs idle: four
+// waves share the steps although some take one or none, since a wave alone walks
+// them one after another. Call us, one wave -> four, 100-token contexts: BF16 head
+// size 128 8 items 8.0 -> 6.1, 256 9.0 -> 8.0 (512 9.7 -> 9.9); 64 8 items 6.6 ->
+// 4.9, 512 8.2 -> 7.5; FP8 128 8 items 7.4 -> 5.6, 256 8.5 -> 7.0. 64 tokens: BF16
+// 128 8 items 6.2 -> 5.6, FP8 256 items 6.9 -> 6.8; 33 tokens 6.1 -> 6.4 (BF16, 256
+// items).
+bool short_split(uint64_t grid, uint32_t steps, uint32_t head_size, bool fp8) {
+  return steps < 8 && steps >= (fp8 ? 5U : 4U) && grid <= (head_size == 64 ? 512U : 256U);
+}
+
+// A 4-wave workgroup of head size 80-128 holds 48 KiB or more: from three items
+// per CU one wave per item runs more of them at once (768 and 960 items of 512
+// and 256 tokens, four waves -> one: head size 128 BF16 35.4 -> 30.7 and 28.6 ->
+// 25.3 us, FP8 27.4 -> 23.3 and 23.2 -> 18.9, 96 FP8 27.4 -> 24.4; 512 items BF16
+// 23.6 -> 26.8), for partitions of up to 512 tokens (800 whole sequences of <= 600
+// tokens, 16-bit 96 36.3 -> 37.4).
+bool single_wave(uint64_t grid, uint32_t steps) { return grid >= 768 && steps <= 32; }
+
 // Head sizes 80, 96 and 112 (16-bit cache, one head tile): the launch shapes
 // of head size 128.
 template <typename QE, bool kFp8, uint32_t kD, int kNt = -1>
 int launch_stream_rot_nt(const DecodeArgs& args, uint64_t grid, uint32_t steps, hipStream_t stream) {
   if (grid >= 4096 || (grid >= 1024 && steps >= 8))
     return launch_stream_group<QE, kFp8, kD, kStreamGroup, kNt>(args, grid, stream);
-  if (steps < 8) return launch_stream<QE, kFp8, 1, 1, kD, kNt>(args, grid, stream);
+  if ((steps < 8 && !short_split(grid, steps, kD, kFp8)) || single_wave(grid, steps))
+    return launch_stream<QE, kFp8, 1, 1, kD, kNt>(args, grid, stream);
   return launch_stream<QE, kFp8, 4, 1, kD, kNt>(args, grid, stream);
 }
 
@@ -3786,7 +3812,13 @@ int launch_f32_stream_nt(const DecodeArgs& args, uint64_t grid, uint32_t steps, 
   constexpr bool kSmall = kD == 64;
   if (grid >= 4096 || (grid >= (kSmall ? 1024 : 2048) && steps >= 8))
     return launch_stream_group<F32Elem, false, kD, kD <= 80 ? 4 : 2, kNt>(args, grid, stream);
-  if (steps < 8 || grid >= 1024) return launch_stream<F32Elem, false, 1, 1, kD, kNt>(args, grid, stream);
+  // Short items share their steps as soon as that saves one (short_split; F32
+  // steps are the longest): 33 tokens, one wave -> four, head size 64 8 items 6.5 ->
+  // 5.3 us, 512 7.4 -> 7.0; 128 8 items 8.8 -> 7.1, 256 9.0 -> 8.1; two waves at 512
+  // items 10.4 -> 9.6.
+  const uint32_t fewest = kSmall ? 3U : 2U;
+  if (steps < fewest || grid >= 1024 || (steps < 8 && grid > 512))
+    return launch_stream<F32Elem, false, 1, 1, kD, kNt>(args, grid, stream);
   if (!kSmall && grid > 256) return launch_stream<F32Elem, false, 2, 1, kD, kNt>(args, grid, stream);
   return launch_stream<F32Elem, false, 4, 1, kD, kNt>(args, grid, stream);
 }
@@ -3978,7 +4010,7 @@ int run_typed(const Problem& p, hipStream_t stream) {
         status = fp8 ? (dense_rows ? launch_stream_group<QE, true, 64, kStreamGroup, 1>(args, grid, stream)
                                    : launch_stream_group<QE, true, 64>(args, grid, stream))
                      : launch_stream_group<QE, false, 64>(args, grid, stream);
-      } else if (steps < 8) {
+      } else if (steps < 8 && !short_split(grid, steps, 64, fp8)) {
         status = fp8 ? (dense_rows ? launch_stream<QE, true, 1, 1, 64, 1>(args, grid, stream)
                                    : launch_stream<QE, true, 1, 1, 64>(args, grid, stream))
                      : launch_stream<QE, false, 1, 1, 64>(args, grid, stream);
@@ -4019,7 +4051,7 @@ int run_typed(const Problem& p, hipStream_t stream) {
                      ? launch_stream_group<QE, false, kDim, 2, -1, false, 1>(args, grid, stream)
                  : p.direct_schedule ? launch_stream_group<QE, false, kDim, kStreamGroup, -1, true>(args, grid, stream)
                                      : launch_stream_group<QE, false>(args, grid, stream);
-      } else if (steps < 8) {
+      } else if ((steps < 8 && !short_split(grid, steps, kDim, fp8)) || single_wave(grid, steps)) {
         status = fp8 ? launch_stream<QE, true, 1>(args, grid, stream) : launch_stream<QE, false, 1>(args, grid, stream);
       } else {
         status = fp8 ? launch_stream<QE, true, 4>(args, grid, stream) : launch_stream<QE, false, 4>(args, grid, stream);
