@@ -1242,8 +1242,8 @@ constexpr int kStreamStages = 2;
 // fill the waves. Call us, two stages -> one: head size 256, single waves, 64
 // x 2048 16-bit 180 -> 171, FP8 98.5 -> 91.9, 44 ragged sequences 111 -> 94.8 and
 // 74.8 -> 62.5; head size 128 16-bit (two-item workgroups) 64 x 512-8192 195.8 ->
-// 190.3, 44 x <= 2874 63.3 -> 52.4, 66 x <= 1015 44.5 -> 42.9, but 1,368 items
-// 43.6 -> 48.8; FP8 pairs 57 x <= 1998 38.1 -> 33.6, 128 x 4096 188.2 -> 187.9.
+// 190.3, 10 x 14000-30000 153.2 -> 149.1, 30 x 32/32 148.7 -> 145.3, but 1,368
+// items 43.6 -> 48.8; FP8 pairs 57 x <= 1998 38.1 -> 33.6, 128 x 4096 188.2 -> 187.9.
 // Head sizes 64-112 keep two (96 NHD ragged 169 -> 175, 64 57 x <= 3000 26.4 ->
 // 39.8).
 constexpr uint64_t kOneStageItems = 2048;
@@ -4044,7 +4044,12 @@ int run_typed(const Problem& p, hipStream_t stream) {
         // The library's own split runs its items in index order with each
         // item's first block IDs loaded alongside its length (C2 decode
         // 18.3-18.5 -> 17.5-17.7 us).
-        const bool one_stage = grid >= kOneStageItems && steps >= 8;
+        // 16-bit one-stage workgroups of two items: not where partitions are
+        // short or few KV heads lie side by side (20 x <= 14438 in 256-token
+        // partitions 111.5 -> 114.7 us, 300 x 12/2 123.4 -> 130.4, 20 x 20/20
+        // 157.3 -> 163.4) nor under 4,096 items (5 x <= 57468 137.9 -> 143.3).
+        const bool one_stage = fp8 ? grid >= kOneStageItems && steps >= 8
+                                   : grid >= 2 * kOneStageItems && steps >= 32 && p.kv_heads % 8 == 0;
         status = fp8 ? (one_stage ? launch_stream_group<QE, true, kDim, kStreamGroup, -1, false, 1>(args, grid, stream)
                                   : launch_stream_group<QE, true>(args, grid, stream))
                  : one_stage && !p.direct_schedule

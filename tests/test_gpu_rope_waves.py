@@ -34,6 +34,14 @@ def test_chunks_of_a_token(dtype, is_neox, encoding, heads, head_size, rotary):
                    maxpos=64, NB=4, bs=4, seed=31)
 
 
+@pytest.mark.parametrize("encoding", ["native", "per-head"])
+@pytest.mark.parametrize("is_neox", [True, False])
+@pytest.mark.parametrize("tokens", [390, 391])  # 799,  801 thousand chunks: either side of the workgroup-per-token rule
+def test_many_chunks_a_token(encoding, is_neox, tokens):
+    check_case(torch.bfloat16, "HND", encoding, is_neox, T=tokens, Hq=32 if is_neox else 16, Hkv=32 if is_neox else 24,
+               D=256, rd=128, maxpos=512, NB=30, bs=16, seed=41)
+
+
 @pytest.mark.parametrize("dtype,cache,tokens,is_neox", [
     (torch.bfloat16, torch.bfloat16, 8201, True), (torch.float16, torch.uint8, 9001, True),
     (torch.bfloat16, torch.uint8, 9001, False), (torch.float32, torch.float32, 4203, False)])
