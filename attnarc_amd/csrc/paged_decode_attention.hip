@@ -1149,8 +1149,9 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a) 
 // Per step: QK^T with v_mfma_f32_16x16x32 (S[token 4g + r][head c] lands in
 // lane (g, c)); PV with v_mfma_f32_16x16x16, whose B operand is exactly that
 // S layout (4 tokens of lane group g) and whose A operand (dims dt*16 + c of
-// tokens 4g + k) is one ds_read_b64_tr_b16 from the 16-bit V tile. FP8 V is
-// converted into that tile once per step; FP8 K is converted as it is read.
+// tokens 4g + k) is one ds_read_b64_tr_b16 from the 16-bit V tile. FP8 caches
+// take steps of 32 tokens and convert K and V as they are read
+// (Fp8StreamDecoder); F32 ones run on F32 MFMA (F32StreamDecoder).
 // ---------------------------------------------------------------------------
 constexpr uint32_t kStep = 16;
 constexpr uint32_t kStepTileBytes = kStep * kTileRowBytes;  // 4 KiB
@@ -1161,9 +1162,7 @@ constexpr uint32_t kStepTileBytes = kStep * kTileRowBytes;  // 4 KiB
 // transposed 8-byte reads are served 32 lanes (rows 4g .. 4g + 3 of two lane
 // groups g, eight rows) at a time over 256 bytes of banks, where rows t and
 // t + 2 share bank offsets at the 128-byte pitch: the permutation differs
-// across each such set of four rows. It also differs in bit 1 between rows
-// 2k and 2k + 1, which keeps the FP8 conversion's 16-byte stores (8 lanes,
-// two rows, 128 bytes of banks at a time) conflict-free.
+// across each such set of four rows.
 template <uint32_t kPitch>
 __host__ __device__ constexpr uint32_t vtile_swizzle(uint32_t t) {
   return kPitch >= 256 ? (t & 7U) << 1 : (((t >> 1) & 3U) ^ (t & 1U)) << 1;
