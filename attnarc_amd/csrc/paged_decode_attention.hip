@@ -153,6 +153,13 @@ struct Fp8Elem {
   }
 };
 
+// A running maximum before its first finite score. Finite, so that scores of
+// -inf (an infinite K element, a product that overflows) weigh
+// exp2(-inf - kNoScore) = 0 where a wave has met no others, instead of
+// exp2(-inf + inf) = NaN; no finite score lies below it, and in the reductions
+// a state without tokens or with none but these keeps l = 0 and O = 0.
+constexpr float kNoScore = -std::numeric_limits<float>::max();
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int offset = 32; offset > 0; offset >>= 1) v += __shfl_xor(v, offset, 64);
@@ -374,7 +381,7 @@ __global__ __launch_bounds__(kVecThreads) void decode_vector_kernel(DecodeArgs a
   float m[kH], l[kH], o[kH][kDvl];
 #pragma unroll
   for (uint32_t h = 0; h < kH; ++h) {
-    m[h] = -INFINITY;
+    m[h] = kNoScore;
     l[h] = 0.0f;
 #pragma unroll
     for (uint32_t j = 0; j < kDvl; ++j) o[h][j] = 0.0f;
@@ -870,7 +877,7 @@ struct MfmaDecoder {
         }
       }
       cmax = head_max(cmax);
-      const float mn = fmaxf(m[ht], cmax);  // finite: every chunk has a valid token
+      const float mn = fmaxf(m[ht], cmax);  // finite: from kNoScore on
       const float alpha = __builtin_amdgcn_exp2f(m[ht] - mn);
       m[ht] = mn;
       float p[8];
@@ -1015,7 +1022,7 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mfma_kernel(DecodeArgs a) 
       const u32x4 w = live ? qw[ht][kc] : u32x4{0U, 0U, 0U, 0U};
       dec.qb[ht][kc] = __builtin_bit_cast(vec8, w);
     }
-    dec.m[ht] = -INFINITY;
+    dec.m[ht] = kNoScore;
     dec.lsum[ht] = 0.0f;
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) dec.acc[ht][dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -1549,7 +1556,7 @@ struct StreamDecoder {
         for (int r = 0; r < 4; ++r) s[ht][r] = t0 + 4 * g + r < p1 ? s[ht][r] : -INFINITY;
       }
       const float cmax = head_max(fmaxf(fmaxf(s[ht][0], s[ht][1]), fmaxf(s[ht][2], s[ht][3])));
-      const float mn = fmaxf(m[ht], cmax);  // finite: every step has a valid token
+      const float mn = fmaxf(m[ht], cmax);  // finite: from kNoScore on
       // Rescale only when some head's maximum moved (exact; usually skipped).
       if (__builtin_amdgcn_ballot_w64(mn > m[ht]) != 0) {
         const float alpha = __builtin_amdgcn_exp2f(m[ht] - mn);
@@ -2042,7 +2049,7 @@ struct Fp8StreamDecoder {
       const f32x4 &x = s[ht][0], &y = s[ht][1];
       const float cmax = head_max(fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])),
                                         fmaxf(fmaxf(y[0], y[1]), fmaxf(y[2], y[3]))));
-      const float mn = fmaxf(m[ht], cmax);  // finite: every step has a valid token
+      const float mn = fmaxf(m[ht], cmax);  // finite: from kNoScore on
       // Rescale only when some head's maximum moved (exact; usually skipped).
       if (__builtin_amdgcn_ballot_w64(mn > m[ht]) != 0) {
         const float alpha = __builtin_amdgcn_exp2f(m[ht] - mn);
@@ -2469,7 +2476,7 @@ __device__ __forceinline__ void pair_publish_empty(uint8_t* tile) {
 }
 
 // Folds the partner's published state into this wave's (m, l, O) by the
-// log-sum-exp identity; this wave's item holds tokens, so m is finite.
+// log-sum-exp identity; this wave's m is finite (kNoScore).
 template <typename Dec>
 __device__ __forceinline__ void pair_combine(const uint8_t* tile, float& m, float& l, f32x4 (&acc)[Dec::kDt]) {
   const uint32_t lane = threadIdx.x & 63U;
@@ -2544,7 +2551,7 @@ __device__ __forceinline__ void stream_item(const DecodeArgs& a, uint8_t* tiles,
 
 #pragma unroll
   for (int ht = 0; ht < kHT; ++ht) {
-    dec.m[ht] = -INFINITY;
+    dec.m[ht] = kNoScore;
     dec.lsum[ht] = 0.0f;
 #pragma unroll
     for (int dt = 0; dt < Dec::kDt; ++dt) dec.acc[ht][dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -2742,7 +2749,7 @@ __device__ __forceinline__ void stream_item_shared(const DecodeArgs& a, uint8_t*
   dec.sl2 = a.score_scale_log2 * k_scale;
 #pragma unroll
   for (int ht = 0; ht < kHTW; ++ht) {
-    dec.m[ht] = -INFINITY;
+    dec.m[ht] = kNoScore;
     dec.lsum[ht] = 0.0f;
 #pragma unroll
     for (int dt = 0; dt < Dec::kDt; ++dt) dec.acc[ht][dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
