@@ -1,0 +1,101 @@
+// Items of the vector RoPE + paged K/V write: which 16-byte chunks each lane of
+// rope_paged_kv_vec_kernel reads. Plain C++, so that a host program can go
+// through every lane of a launch.
+#pragma once
+
+#include <cstdint>
+
+#ifdef __HIPCC__
+#define LOOM_ROPE_HD __host__ __device__ __forceinline__
+#else
+#define LOOM_ROPE_HD inline
+#endif
+
+namespace loom_hip_rope {
+
+// Divisions of the item decode as multiplications by rounded inverses.
+struct VecDivisors {
+  uint32_t waves_per_token;
+  uint32_t token_inverse;      // floor(2^32 / waves_per_token), saturated
+  uint32_t rot, tail, value;   // floor(2^32 / chunks) + 1: exact below 2^16 items a token; 0: divide
+};
+
+// Chunks of a head's row and their counts.
+struct VecCounts {
+  uint32_t query_heads, kv_heads;
+  uint32_t rot_items, tail_chunks, value_chunks;  // a head's rotary items, K tail chunks and V chunks
+};
+
+inline VecDivisors vec_divisors(uint64_t query_heads, uint64_t kv_heads, uint64_t rot_items, uint64_t tail_chunks,
+                                uint64_t value_chunks) {
+  const uint64_t items = query_heads * rot_items + kv_heads * (rot_items + tail_chunks + value_chunks);
+  const uint64_t waves_per_token = (items + 63) / 64;
+  // chunks == 1 would need 2^32 + 1: divided by one instead
+  auto inverse = [&](uint64_t chunks) -> uint32_t {
+    return chunks > 1 && items < (1ULL << 16) ? static_cast<uint32_t>((1ULL << 32) / chunks + 1U) : 0U;
+  };
+  const uint64_t token_inverse = (1ULL << 32) / waves_per_token;
+  return {static_cast<uint32_t>(waves_per_token),
+          static_cast<uint32_t>(token_inverse > 0xffffffffULL ? 0xffffffffULL : token_inverse), inverse(rot_items),
+          inverse(tail_chunks), inverse(value_chunks)};
+}
+
+LOOM_ROPE_HD uint32_t mul_high(uint32_t a, uint32_t b) {
+  return static_cast<uint32_t>((static_cast<uint64_t>(a) * b) >> 32);
+}
+
+// The token of wave `unit` of the launch, and the wave's place in it.
+LOOM_ROPE_HD uint32_t vec_token(const VecDivisors& div, uint32_t unit, uint32_t* wave) {
+  uint32_t token = mul_high(unit, div.token_inverse);  // unit / waves_per_token, or one less
+  *wave = unit - token * div.waves_per_token;
+  if (*wave >= div.waves_per_token) {
+    ++token;
+    *wave -= div.waves_per_token;
+  }
+  return token;
+}
+
+enum : uint32_t { kQueryRotary, kKeyRotary, kKeyTail, kValueChunk, kNoItem };
+
+struct VecItem {
+  uint32_t kind, head, chunk;
+};
+
+// Item `item` of a token: its rotary items of Q, then of K, then K tail and V
+// chunks.
+LOOM_ROPE_HD VecItem vec_item(const VecCounts& n, const VecDivisors& div, uint32_t item) {
+  const uint32_t q_items = n.query_heads * n.rot_items;
+  const uint32_t k_items = n.kv_heads * n.rot_items;
+  const uint32_t t_items = n.kv_heads * n.tail_chunks;
+  uint32_t r = item, kind = kQueryRotary, per = n.rot_items, inverse = div.rot;
+  if (r >= q_items) {
+    r -= q_items;
+    kind = kKeyRotary;
+    if (r >= k_items) {
+      r -= k_items;
+      kind = kKeyTail;
+      per = n.tail_chunks;
+      inverse = div.tail;
+      if (r >= t_items) {
+        r -= t_items;
+        kind = kValueChunk;
+        per = n.value_chunks;
+        inverse = div.value;
+        if (r >= n.kv_heads * n.value_chunks) return {kNoItem, 0, 0};
+      }
+    }
+  }
+  const uint32_t head = inverse != 0 ? mul_high(r, inverse) : r / per;
+  return {kind, head, r - head * per};
+}
+
+// Whether the token of slot entry `slot` (-1: it has none) goes to the caches.
+LOOM_ROPE_HD bool vec_writes(int64_t slot, uint32_t num_blocks, uint32_t block_size) {
+  return slot >= 0 && static_cast<uint64_t>(slot) < static_cast<uint64_t>(num_blocks) * block_size;
+}
+
+// Whether a lane reads its item's source row. K tail and V serve the caches
+// only; V need not hold a row for a token that does not go there.
+LOOM_ROPE_HD bool vec_reads(uint32_t kind, bool writes) { return kind <= kKeyRotary || writes; }
+
+}  // namespace loom_hip_rope

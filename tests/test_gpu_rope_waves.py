@@ -71,3 +71,29 @@ def test_large_calls_equal_small_ones(dtype, cache, tokens, is_neox):
 
     (rows, kv), (want_rows, want_kv) = write(1), write(0)
     assert torch.equal(rows, want_rows) and torch.equal(kv, want_kv)
+
+
+@pytest.mark.parametrize("is_neox", [True, False])
+@pytest.mark.parametrize("cache_tokens", [0, 1, 6])
+def test_value_rows_end_with_the_slots(is_neox, cache_tokens):
+    # V rows exist for the tokens that have a slot entry only
+    tokens, hq, hkv, d, rd, bs = 9, 12, 2, 64, 32, 4
+    gen = torch.Generator(device=DEV).manual_seed(11)
+    q0, k0, v = (torch.randn((tokens, h, d), generator=gen, device=DEV).bfloat16() for h in (hq, hkv, hkv))
+    pos = torch.randint(0, 64, (tokens,), generator=gen, device=DEV)
+    cs = cos_sin_cache(64, rd, torch.bfloat16)
+    slots = torch.randperm(6 * bs, generator=gen, device=DEV)[:tokens]
+
+    def write(value, mapping):
+        q, k = q0.clone(), k0.clone()
+        kc, vc = (torch.full((6, bs, hkv, d), -3.0, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+        ops.rope_paged_kv_write_strided(q, k, value, pos, cs, kc, vc, None, None, mapping, num_blocks=6, block_size=bs,
+                                        key_cache_strides=kc.stride()[:3], value_cache_strides=vc.stride()[:3],
+                                        is_neox=is_neox)
+        torch.cuda.synchronize()
+        return q, k, kc, vc
+
+    padded = torch.where(torch.arange(tokens, device=DEV) < cache_tokens, slots, -1)
+    want = write(v, padded)
+    got = write(v[: max(cache_tokens, 1)].clone(), slots[:cache_tokens].clone() if cache_tokens else None)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
