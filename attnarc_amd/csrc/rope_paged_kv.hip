@@ -381,8 +381,6 @@ __global__ __launch_bounds__(kRopeThreads) void rope_paged_kv_vec_kernel(RopeArg
 // F32 527 tokens 13.5 -> 12.1; but 64/8 (704 chunks) 700 tokens 8.7 -> 9.5 and 200
 // tokens of 32/32 at 256 8.4 -> 9.0.
 constexpr uint32_t kTokenUnroll = 2;
-constexpr uint64_t kTokenKernelChunks = 1024;
-constexpr uint64_t kTokenKernelTotal = 800000;
 
 template <typename E, bool kFp8, bool kNeox>
 __global__ __launch_bounds__(kRopeThreads) void rope_paged_kv_token_kernel(RopeArgs a, uint32_t splits) {
@@ -510,13 +508,6 @@ __global__ __launch_bounds__(kRopeThreads) void rope_paged_kv_token_kernel(RopeA
   }
 }
 
-// Calls that touch more than this many bytes take the non-temporal hint on the
-// rows and the caches: past it the 256 MiB Infinity Cache keeps little of them
-// for the next kernel. Us without / with the hint at 32/8 heads, head size 128:
-// BF16 cache 134 MB 22.8 / 24.5, 161 MB 27.9 / 28.8, 188 MB 34.3 / 33.1, 215 MB
-// 41.6 / 37.4, 323 MB 62.7 / 54.7; FP8 124 MB 22.9 / 24.6, 199 MB 37.8 / 35.4.
-constexpr uint64_t kNtBytes = 192ULL << 20;
-
 template <typename E, bool kFp8, bool kNeox>
 void launch_vec(const RopeArgs& args, uint32_t grid, const VecDivisors& div, bool nt, hipStream_t s) {
   if (nt) {
@@ -594,26 +585,18 @@ int rope_write(void* query, void* key, const void* value, const int64_t* positio
       value_cache_head_stride % N == 0 && aligned(query, 16) && aligned(key, 16) && aligned(value, 16) &&
       aligned(cos_sin_cache, 16) && aligned(key_cache, N * cache_elem) && aligned(value_cache, N * cache_elem);
   const uint64_t rot_items = is_neox ? rotary_dim / 2 / N : rotary_dim / N;
-  const uint64_t max_items = static_cast<uint64_t>(query_heads) * rot_items +
-                             static_cast<uint64_t>(kv_heads) * (rot_items + (head_size - rotary_dim) / N +
-                                                                value_head_size / N);
-  const uint64_t waves_per_token = (max_items + 63) / 64;
-  const uint64_t waves = tokens * waves_per_token;
-  if (vec_ok && waves <= static_cast<uint64_t>(std::numeric_limits<int>::max())) {
-    const uint64_t token_bytes =
-        2ULL * (query_heads + kv_heads) * rotary_dim * sizeof(typename E::T) +
-        static_cast<uint64_t>(kv_heads) * (head_size - rotary_dim + value_head_size) * sizeof(typename E::T) +
-        static_cast<uint64_t>(kv_heads) * (head_size + value_head_size) * cache_elem;
-    const bool nt = token_bytes * tokens > kNtBytes;
-    const uint32_t grid = static_cast<uint32_t>((waves + kRopeRowsPerGroup - 1) / kRopeRowsPerGroup);
-    const VecDivisors div = vec_divisors(query_heads, kv_heads, rot_items, (head_size - rotary_dim) / N,
-                                         value_head_size / N);
-    if (!nt && max_items >= kTokenKernelChunks && max_items * tokens >= kTokenKernelTotal) {
-      const uint64_t max_splits = (max_items + kRopeThreads - 1) / kRopeThreads;
-      uint64_t splits = (2048 + tokens - 1) / tokens;  // cover the chip
-      if (splits > max_splits) splits = max_splits;
-      const dim3 tgrid(static_cast<uint32_t>(tokens * splits)), block(kRopeThreads);
-      const uint32_t sp = static_cast<uint32_t>(splits);
+  const uint64_t tail_chunks = (head_size - rotary_dim) / N, value_chunks = value_head_size / N;
+  const uint64_t token_bytes =
+      2ULL * (static_cast<uint64_t>(query_heads) + kv_heads) * rotary_dim * sizeof(typename E::T) +
+      static_cast<uint64_t>(kv_heads) * (head_size - rotary_dim + value_head_size) * sizeof(typename E::T) +
+      static_cast<uint64_t>(kv_heads) * (head_size + value_head_size) * cache_elem;
+  const WritePlan plan = vec_ok ? write_plan({tokens, query_heads, kv_heads, rot_items, tail_chunks, value_chunks,
+                                              token_bytes * tokens})
+                                : WritePlan{WriteKernel::kGeneral, false, 0, 0};
+  if (plan.kernel != WriteKernel::kGeneral) {
+    if (plan.kernel == WriteKernel::kTokens) {
+      const dim3 tgrid(plan.grid), block(kRopeThreads);
+      const uint32_t sp = plan.splits;
       if (fp8) {
         if (is_neox) hipLaunchKernelGGL((rope_paged_kv_token_kernel<E, true, true>), tgrid, block, 0, s, args, sp);
         else hipLaunchKernelGGL((rope_paged_kv_token_kernel<E, true, false>), tgrid, block, 0, s, args, sp);
@@ -621,12 +604,15 @@ int rope_write(void* query, void* key, const void* value, const int64_t* positio
         if (is_neox) hipLaunchKernelGGL((rope_paged_kv_token_kernel<E, false, true>), tgrid, block, 0, s, args, sp);
         else hipLaunchKernelGGL((rope_paged_kv_token_kernel<E, false, false>), tgrid, block, 0, s, args, sp);
       }
-    } else if (fp8) {
-      if (is_neox) launch_vec<E, true, true>(args, grid, div, nt, s);
-      else launch_vec<E, true, false>(args, grid, div, nt, s);
     } else {
-      if (is_neox) launch_vec<E, false, true>(args, grid, div, nt, s);
-      else launch_vec<E, false, false>(args, grid, div, nt, s);
+      const VecDivisors div = vec_divisors(query_heads, kv_heads, rot_items, tail_chunks, value_chunks);
+      if (fp8) {
+        if (is_neox) launch_vec<E, true, true>(args, plan.grid, div, plan.nt, s);
+        else launch_vec<E, true, false>(args, plan.grid, div, plan.nt, s);
+      } else {
+        if (is_neox) launch_vec<E, false, true>(args, plan.grid, div, plan.nt, s);
+        else launch_vec<E, false, false>(args, plan.grid, div, plan.nt, s);
+      }
     }
     if (hipGetLastError() != hipSuccess) return fail(LOOM_HIP_LAUNCH_ERROR, "RoPE+paged-KV kernel launch failed");
     loom_hip_detail::count_launch(LOOM_HIP_ROPE_PAGED_KV_WRITE);

@@ -1,6 +1,6 @@
-// Items of the vector RoPE + paged K/V write: which 16-byte chunks each lane of
-// rope_paged_kv_vec_kernel reads. Plain C++, so that a host program can go
-// through every lane of a launch.
+// The RoPE + paged K/V write as a launch: which kernel a call takes, and which
+// 16-byte chunks each lane of rope_paged_kv_vec_kernel reads. Plain C++, so that a
+// host program can look at any call and go through every lane of a launch.
 #pragma once
 
 #include <cstdint>
@@ -97,5 +97,58 @@ LOOM_ROPE_HD bool vec_writes(int64_t slot, uint32_t num_blocks, uint32_t block_s
 // Whether a lane reads its item's source row. K tail and V serve the caches
 // only; V need not hold a row for a token that does not go there.
 LOOM_ROPE_HD bool vec_reads(uint32_t kind, bool writes) { return kind <= kKeyRotary || writes; }
+
+enum class WriteKernel : uint32_t {
+  kGeneral,  // rope_paged_kv_kernel
+  kWaves,    // rope_paged_kv_vec_kernel
+  kTokens,   // rope_paged_kv_token_kernel
+};
+
+struct WriteShape {
+  uint64_t tokens, query_heads, kv_heads;
+  uint64_t rot_items, tail_chunks, value_chunks;  // a head's, as in VecCounts
+  uint64_t bytes;                                 // that the call touches
+};
+
+struct WritePlan {
+  WriteKernel kernel;
+  bool nt;        // kWaves: non-temporal hint
+  uint32_t grid;  // workgroups
+  uint32_t splits;  // kTokens: workgroups a token
+};
+
+// Calls that touch more than this many bytes take the non-temporal hint on the
+// rows and the caches: past it the 256 MiB Infinity Cache keeps little of them
+// for the next kernel. Us without / with the hint at 32/8 heads, head size 128:
+// BF16 cache 134 MB 22.8 / 24.5, 161 MB 27.9 / 28.8, 188 MB 34.3 / 33.1, 215 MB
+// 41.6 / 37.4, 323 MB 62.7 / 54.7; FP8 124 MB 22.9 / 24.6, 199 MB 37.8 / 35.4.
+constexpr uint64_t kNtBytes = 192ULL << 20;
+
+// The workgroup-per-token kernel: many chunks a token, and enough of them to fill
+// the chip (figures at the kernel).
+constexpr uint64_t kTokenKernelChunks = 1024;
+constexpr uint64_t kTokenKernelTotal = 800000;
+
+// The kernel of a call whose rows, strides and bases are whole 16-byte chunks.
+// Both vector kernels number a token's items in 32 bits, and a launch takes fewer
+// than 2^32 threads: past either the call goes to the other one, or to the
+// general kernel.
+inline WritePlan write_plan(const WriteShape& s) {
+  constexpr uint64_t kMaxItems = 1ULL << 31, kThreads = 256, kMaxGroups = 0xffffffffULL / kThreads;
+  const uint64_t items = s.query_heads * s.rot_items + s.kv_heads * (s.rot_items + s.tail_chunks + s.value_chunks);
+  const WritePlan general{WriteKernel::kGeneral, false, 0, 0};
+  if (items > kMaxItems) return general;
+  const uint64_t wave_groups = (s.tokens * ((items + 63) / 64) + 3) / 4;
+  const uint64_t max_splits = (items + kThreads - 1) / kThreads;
+  uint64_t splits = (2048 + s.tokens - 1) / s.tokens;  // cover the chip
+  if (splits > max_splits) splits = max_splits;
+  const bool waves_fit = wave_groups <= kMaxGroups, tokens_fit = s.tokens * splits <= kMaxGroups;
+  if (!waves_fit && !tokens_fit) return general;
+  const bool nt = s.bytes > kNtBytes;
+  const bool by_token = !nt && items >= kTokenKernelChunks && items * s.tokens >= kTokenKernelTotal;
+  if ((by_token && tokens_fit) || !waves_fit)
+    return {WriteKernel::kTokens, false, static_cast<uint32_t>(s.tokens * splits), static_cast<uint32_t>(splits)};
+  return {WriteKernel::kWaves, nt, static_cast<uint32_t>(wave_groups), 0};
+}
 
 }  // namespace loom_hip_rope

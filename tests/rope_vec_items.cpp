@@ -1,7 +1,18 @@
-// Walks every lane of a launch of the vector RoPE + K/V write on the host and
-// counts how often it reads each item's source: counts[token][query rotary | key
-// rotary | key tail | value].
+// The vector RoPE + K/V write looked at on the host.
 #include "rope_vec_items.h"
+
+// out: kernel, non-temporal, workgroups, workgroups a token.
+extern "C" void plan_of(uint64_t tokens, uint64_t query_heads, uint64_t kv_heads, uint64_t rot_items,
+                        uint64_t tail_chunks, uint64_t value_chunks, uint64_t bytes, uint32_t* out) {
+  const auto p = loom_hip_rope::write_plan({tokens, query_heads, kv_heads, rot_items, tail_chunks, value_chunks, bytes});
+  out[0] = static_cast<uint32_t>(p.kernel);
+  out[1] = p.nt;
+  out[2] = p.grid;
+  out[3] = p.splits;
+}
+
+// Walks every lane of a launch and counts how often it reads each item's source:
+// counts[token][query rotary | key rotary | key tail | value].
 
 extern "C" int walk_items(uint32_t tokens, uint32_t cache_tokens, const int64_t* slots, uint32_t num_blocks,
                           uint32_t block_size, uint32_t query_heads, uint32_t kv_heads, uint32_t rot_items,

@@ -1,4 +1,4 @@
-"""The lanes of the vector RoPE + paged K/V write, walked on the host.
+"""The launches of the vector RoPE + paged K/V write, and their lanes, walked on the host.
 
 Each launch has to read every rotary item of every token once, and the K tail
 and V chunks of exactly the tokens that have a slot: V rows past cache_tokens
@@ -17,13 +17,16 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
+GENERAL, WAVES, TOKENS = range(3)
+
+
 @pytest.fixture(scope="module")
-def walk(tmp_path_factory):
+def shim(tmp_path_factory):
     out = str(tmp_path_factory.mktemp("rope") / "rope_vec_items.so")
     subprocess.run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC",
                     f"-I{os.path.join(ROOT, 'attnarc_amd', 'csrc')}",
                     os.path.join(ROOT, "tests", "rope_vec_items.cpp"), "-o", out], check=True)
-    return ctypes.CDLL(out).walk_items
+    return ctypes.CDLL(out)
 
 
 @pytest.mark.parametrize("cache_tokens", [0, 1, 5, 9])
@@ -36,16 +39,43 @@ def walk(tmp_path_factory):
     (71, 1, 5, 0, 10),     # chunk counts that no power of two divides
     (64, 64, 64, 0, 1000),  # over 2^16 items a token: plain division
 ])
-def test_every_item_once(walk, cache_tokens, query_heads, kv_heads, rot, tail, value):
+def test_every_item_once(shim, cache_tokens, query_heads, kv_heads, rot, tail, value):
     tokens = 9
     slots = np.array([3, -1, 0, 32, 31, 7, -5, 1, 9], dtype=np.int64)  # 2 blocks of 16 tokens
     rotary = (query_heads + kv_heads) * rot
     items = rotary + kv_heads * (tail + value)
     counts = np.zeros((tokens, items), dtype=np.uint8)
-    status = walk(tokens, cache_tokens, slots.ctypes.data_as(ctypes.c_void_p), 2, 16, query_heads, kv_heads, rot, tail,
-                  value, counts.ctypes.data_as(ctypes.c_void_p))
+    status = shim.walk_items(tokens, cache_tokens, slots.ctypes.data_as(ctypes.c_void_p), 2, 16, query_heads,
+                             kv_heads, rot, tail, value, counts.ctypes.data_as(ctypes.c_void_p))
     assert status == 0
     want = np.zeros_like(counts)
     want[:, :rotary] = 1
     want[[t for t in range(cache_tokens) if 0 <= slots[t] < 32], rotary:] = 1
     np.testing.assert_array_equal(counts, want)
+
+
+def _plan(shim, tokens, query_heads, kv_heads, rot, tail, value, nbytes=0):
+    out = (ctypes.c_uint32 * 4)()
+    shim.plan_of(*(ctypes.c_uint64(x) for x in (tokens, query_heads, kv_heads, rot, tail, value, nbytes)), out)
+    return tuple(out)
+
+
+@pytest.mark.parametrize("tokens,query_heads,rot,kernel", [
+    (1, (1 << 31) - 2, 1, TOKENS),     # 2^31 chunks a token
+    (1, (1 << 31) - 1, 1, GENERAL),    # one more
+    (1, (1 << 32) - 1, 1, GENERAL),    # numbers of 2^32 and more would wrap
+    (1, (1 << 32) - 1, 64, GENERAL),
+    (20_000_000, 62, 1, WAVES),        # 64 chunks a token
+    (16_777_215, 254, 1, WAVES),       # 256 chunks: one workgroup a token, the last launch that fits
+    (16_777_216, 254, 1, GENERAL),     # 2^32 threads either way
+    (13_500_000, 318, 1, TOKENS),      # 320 chunks: 80 lanes' waves would be 1.3 workgroups a token
+    (13_421_772, 318, 1, WAVES),
+    (16_777_216, 318, 1, GENERAL),
+])
+def test_launch_and_index_limits(shim, tokens, query_heads, rot, kernel):
+    got, _, groups, splits = _plan(shim, tokens, query_heads, 1, rot, 0, 1)
+    assert got == kernel
+    if got != GENERAL:
+        items = (query_heads + 1) * rot + 1
+        need = -(-tokens * -(-items // 64) // 4) if got == WAVES else tokens * splits
+        assert groups == need and groups * 256 < 1 << 32
