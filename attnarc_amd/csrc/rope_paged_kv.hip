@@ -374,12 +374,8 @@ __global__ __launch_bounds__(kRopeThreads) void rope_paged_kv_vec_kernel(RopeArg
 
 // The same items a workgroup per (token, split), kTokenUnroll a thread, all of
 // their loads issued together after the token's position. Kept where it is the
-// faster one: many chunks a token (kTokenKernelChunks) and enough of them to fill
-// the chip, in the Infinity Cache, where half as many waves matter more than
-// earlier loads. Us, a wave per 64 chunks -> this: 32/32 heads at 256, 631 tokens,
-// FP8 18.5 -> 14.7, BF16 18.2 -> 14.2; 32/32 at 128, 1,500 tokens FP8 21.4 -> 17.7,
-// F32 527 tokens 13.5 -> 12.1; but 64/8 (704 chunks) 700 tokens 8.7 -> 9.5 and 200
-// tokens of 32/32 at 256 8.4 -> 9.0.
+// faster one (prefers_tokens): where no thread of it is left idle, and in the
+// Infinity Cache, where half as many waves matter more than earlier loads.
 constexpr uint32_t kTokenUnroll = 2;
 
 template <typename E, bool kFp8, bool kNeox>
@@ -590,8 +586,15 @@ int rope_write(void* query, void* key, const void* value, const int64_t* positio
       2ULL * (static_cast<uint64_t>(query_heads) + kv_heads) * rotary_dim * sizeof(typename E::T) +
       static_cast<uint64_t>(kv_heads) * (head_size - rotary_dim + value_head_size) * sizeof(typename E::T) +
       static_cast<uint64_t>(kv_heads) * (head_size + value_head_size) * cache_elem;
+  // A token's heads lie side by side in an NHD cache; otherwise each is a row of its own.
+  auto cache_lines = [&](uint64_t head_stride, uint64_t row) {
+    return head_stride == row || row * cache_elem % 128 == 0;
+  };
+  const bool whole_lines = static_cast<uint64_t>(rotary_dim) * sizeof(typename E::T) % 128 == 0 &&
+                           cache_lines(key_cache_head_stride, head_size) &&
+                           cache_lines(value_cache_head_stride, value_head_size);
   const WritePlan plan = vec_ok ? write_plan({tokens, query_heads, kv_heads, rot_items, tail_chunks, value_chunks,
-                                              token_bytes * tokens})
+                                              token_bytes * tokens, fp8, whole_lines})
                                 : WritePlan{WriteKernel::kGeneral, false, 0, 0};
   if (plan.kernel != WriteKernel::kGeneral) {
     if (plan.kernel == WriteKernel::kTokens) {

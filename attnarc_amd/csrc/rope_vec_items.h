@@ -108,6 +108,8 @@ struct WriteShape {
   uint64_t tokens, query_heads, kv_heads;
   uint64_t rot_items, tail_chunks, value_chunks;  // a head's, as in VecCounts
   uint64_t bytes;                                 // that the call touches
+  bool fp8;                                       // the caches hold FP8
+  bool whole_lines;  // rotated rows and cache rows are whole 128-byte lines
 };
 
 struct WritePlan {
@@ -117,17 +119,32 @@ struct WritePlan {
   uint32_t splits;  // kTokens: workgroups a token
 };
 
-// Calls that touch more than this many bytes take the non-temporal hint on the
-// rows and the caches: past it the 256 MiB Infinity Cache keeps little of them
-// for the next kernel. Us without / with the hint at 32/8 heads, head size 128:
-// BF16 cache 134 MB 22.8 / 24.5, 161 MB 27.9 / 28.8, 188 MB 34.3 / 33.1, 215 MB
-// 41.6 / 37.4, 323 MB 62.7 / 54.7; FP8 124 MB 22.9 / 24.6, 199 MB 37.8 / 35.4.
+// Calls of whole 128-byte lines that touch more than this many bytes take the
+// non-temporal hint on the rows and the caches: past it the 256 MiB Infinity
+// Cache keeps little of them for the next kernel. Us without / with the hint at
+// 32/8 heads, head size 128: BF16 cache 134 MB 22.8 / 24.5, 161 MB 27.9 / 28.8, 188
+// MB 34.3 / 33.1, 215 MB 41.6 / 37.4, 323 MB 62.7 / 54.7; FP8 124 MB 22.9 / 24.6,
+// 199 MB 37.8 / 35.4. Stores of part of a line are not joined under the hint: 32/8
+// heads, head size 96, half rotary, 300 MB 100 / 135.
 constexpr uint64_t kNtBytes = 192ULL << 20;
 
-// The workgroup-per-token kernel: many chunks a token, and enough of them to fill
-// the chip (figures at the kernel).
-constexpr uint64_t kTokenKernelChunks = 1024;
-constexpr uint64_t kTokenKernelTotal = 800000;
+// The workgroup-per-token kernel (two items a thread) against waves of 64 chunks:
+//   - 480 to 512 chunks a token, or a multiple of 512, leave it no idle thread.
+//     From 24 MiB on. Us, waves -> workgroups a token: 16/16 heads, head size 128,
+//     30 MB 8.7 -> 8.5 (12 MB 4.4 -> 5.0), 100 MB 22.7 -> 20.6; 32/32 at 128, half
+//     rotary, FP8 300 MB 94 -> 74; 32/32 at 64, 300 MB 69 -> 60; but 768 chunks
+//     (32/32 at 96, half rotary) waves by 2-9%.
+//   - native caches from 256 chunks a token, 44 to 186 MiB, mostly in the Infinity
+//     Cache: 20/20 at 80, 100 MB 19.6 -> 18.2, 32/8 at 128, 100 MB 19.0 -> 18.1 (300
+//     MB: waves by 4-11%), 32/8 at 80, 30 MB 8.4 against 11.3 (waves), FP8 at 80 25.3
+//     against 25.8 (waves).
+constexpr uint64_t kFullTokenBytes = 24ULL << 20;
+constexpr uint64_t kNativeTokenChunks = 256, kNativeTokenBytes = 44ULL << 20, kNativeTokenMaxBytes = 186ULL << 20;
+
+inline bool prefers_tokens(const WriteShape& s, uint64_t items) {
+  if (items % 512 == 0 || (items >= 480 && items < 512)) return s.bytes > kFullTokenBytes;
+  return !s.fp8 && items >= kNativeTokenChunks && s.bytes > kNativeTokenBytes && s.bytes <= kNativeTokenMaxBytes;
+}
 
 // The kernel of a call whose rows, strides and bases are whole 16-byte chunks.
 // Both vector kernels number a token's items in 32 bits, and a launch takes fewer
@@ -144,11 +161,9 @@ inline WritePlan write_plan(const WriteShape& s) {
   if (splits > max_splits) splits = max_splits;
   const bool waves_fit = wave_groups <= kMaxGroups, tokens_fit = s.tokens * splits <= kMaxGroups;
   if (!waves_fit && !tokens_fit) return general;
-  const bool nt = s.bytes > kNtBytes;
-  const bool by_token = !nt && items >= kTokenKernelChunks && items * s.tokens >= kTokenKernelTotal;
-  if ((by_token && tokens_fit) || !waves_fit)
+  if ((prefers_tokens(s, items) && tokens_fit) || !waves_fit)
     return {WriteKernel::kTokens, false, static_cast<uint32_t>(s.tokens * splits), static_cast<uint32_t>(splits)};
-  return {WriteKernel::kWaves, nt, static_cast<uint32_t>(wave_groups), 0};
+  return {WriteKernel::kWaves, s.whole_lines && s.bytes > kNtBytes, static_cast<uint32_t>(wave_groups), 0};
 }
 
 }  // namespace loom_hip_rope

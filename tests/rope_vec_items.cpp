@@ -3,8 +3,10 @@
 
 // out: kernel, non-temporal, workgroups, workgroups a token.
 extern "C" void plan_of(uint64_t tokens, uint64_t query_heads, uint64_t kv_heads, uint64_t rot_items,
-                        uint64_t tail_chunks, uint64_t value_chunks, uint64_t bytes, uint32_t* out) {
-  const auto p = loom_hip_rope::write_plan({tokens, query_heads, kv_heads, rot_items, tail_chunks, value_chunks, bytes});
+                        uint64_t tail_chunks, uint64_t value_chunks, uint64_t bytes, uint64_t fp8, uint64_t whole_lines,
+                        uint32_t* out) {
+  const auto p = loom_hip_rope::write_plan({tokens, query_heads, kv_heads, rot_items, tail_chunks, value_chunks, bytes,
+                                            fp8 != 0, whole_lines != 0});
   out[0] = static_cast<uint32_t>(p.kernel);
   out[1] = p.nt;
   out[2] = p.grid;

@@ -36,10 +36,16 @@ def test_chunks_of_a_token(dtype, is_neox, encoding, heads, head_size, rotary):
 
 @pytest.mark.parametrize("encoding", ["native", "per-head"])
 @pytest.mark.parametrize("is_neox", [True, False])
-@pytest.mark.parametrize("tokens", [390, 391])  # 799,  801 thousand chunks: either side of the workgroup-per-token rule
+@pytest.mark.parametrize("tokens", [279, 280, 341, 342, 390, 391])  # NeoX: 24 MiB from 280 (FP8: 342), a workgroup a token
 def test_many_chunks_a_token(encoding, is_neox, tokens):
     check_case(torch.bfloat16, "HND", encoding, is_neox, T=tokens, Hq=32 if is_neox else 16, Hkv=32 if is_neox else 24,
                D=256, rd=128, maxpos=512, NB=30, bs=16, seed=41)
+
+
+@pytest.mark.parametrize("tokens", [1732, 1733])  # 44 MiB from 1,733: a workgroup a token over native caches
+def test_native_caches_of_448_chunks(tokens):
+    check_case(torch.bfloat16, "NHD", "native", True, T=tokens, Hq=32, Hkv=8, D=128, rd=128, maxpos=512, NB=120, bs=16,
+               seed=43)
 
 
 @pytest.mark.parametrize("dtype,cache,tokens,is_neox", [

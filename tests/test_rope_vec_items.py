@@ -54,14 +54,15 @@ def test_every_item_once(shim, cache_tokens, query_heads, kv_heads, rot, tail, v
     np.testing.assert_array_equal(counts, want)
 
 
-def _plan(shim, tokens, query_heads, kv_heads, rot, tail, value, nbytes=0):
+def _plan(shim, tokens, query_heads, kv_heads, rot, tail, value, nbytes=0, fp8=0, whole_lines=1):
     out = (ctypes.c_uint32 * 4)()
-    shim.plan_of(*(ctypes.c_uint64(x) for x in (tokens, query_heads, kv_heads, rot, tail, value, nbytes)), out)
+    shim.plan_of(*(ctypes.c_uint64(x) for x in (tokens, query_heads, kv_heads, rot, tail, value, nbytes, fp8,
+                                                whole_lines)), out)
     return tuple(out)
 
 
 @pytest.mark.parametrize("tokens,query_heads,rot,kernel", [
-    (1, (1 << 31) - 2, 1, TOKENS),     # 2^31 chunks a token
+    (1, (1 << 31) - 2, 1, WAVES),      # 2^31 chunks a token
     (1, (1 << 31) - 1, 1, GENERAL),    # one more
     (1, (1 << 32) - 1, 1, GENERAL),    # numbers of 2^32 and more would wrap
     (1, (1 << 32) - 1, 64, GENERAL),
@@ -79,3 +80,27 @@ def test_launch_and_index_limits(shim, tokens, query_heads, rot, kernel):
         items = (query_heads + 1) * rot + 1
         need = -(-tokens * -(-items // 64) // 4) if got == WAVES else tokens * splits
         assert groups == need and groups * 256 < 1 << 32
+
+
+@pytest.mark.parametrize("heads,head_size,rotary,fp8,tokens,kernel,hint", [
+    # Shapes that were slower on the other kernel, or with the hint (BF16 rows): us at each line of the rule, chosen
+    # against the other.
+    ((32, 32), 64, 64, 0, 10463, TOKENS, 0),    # 60 against 69 (73 with the hint)
+    ((32, 32), 128, 64, 1, 8138, TOKENS, 0),    # 73 against 93 (95)
+    ((16, 16), 128, 64, 0, 8000, TOKENS, 0),    # 32 against 34
+    ((20, 20), 80, 80, 0, 4464, TOKENS, 0),     # 18.2 against 19.6
+    ((32, 8), 128, 128, 0, 3756, TOKENS, 0),    # 18.1 against 19.0
+    ((32, 8), 128, 128, 1, 4000, WAVES, 0),     # 18.8 against 19.6
+    ((16, 16), 128, 128, 0, 418, WAVES, 0),     # 4.4 against 5.0
+    ((32, 8), 80, 80, 0, 1802, WAVES, 0),       # 8.4 against 11.3
+    ((12, 2), 64, 64, 0, 32768, WAVES, 0),      # 28 against 51
+    ((32, 8), 96, 48, 0, 22977, WAVES, 0),      # 100 against 135 with the hint
+    ((8, 8), 96, 48, 0, 35511, WAVES, 0),       # 87 against 124 with the hint
+    ((32, 8), 128, 128, 0, 32768, WAVES, 1),    # 149 against 168
+])
+def test_kernel_and_hint(shim, heads, head_size, rotary, fp8, tokens, kernel, hint):
+    hq, hkv = heads
+    rot, tail, value = rotary // 2 // 8, (head_size - rotary) // 8, head_size // 8
+    row = 2 * (hq + hkv) * rotary * 2 + hkv * (2 * head_size - rotary) * 2 + 2 * hkv * head_size * (1 if fp8 else 2)
+    got = _plan(shim, tokens, hq, hkv, rot, tail, value, row * tokens, fp8, rotary * 2 % 128 == 0)
+    assert got[:2] == (kernel, hint)
