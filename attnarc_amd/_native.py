@@ -174,16 +174,27 @@ _CALL_ENTRY_POINTS = (
 )
 
 
+class _PythonCalls:
+    """Takes no call: ops.py's own path does."""
+
+    def decode_extended(self, *args):
+        return None
+
+    decode_views = rope_write = decode_extended
+
+
 def calls():
-    """The native call module (csrc/host_calls.cpp), bound to the loaded library's entry points."""
+    """The native call module (csrc/host_calls.cpp), bound to the loaded library's entry points, or a stand-in that
+    leaves every call to ops.py where none was built for this interpreter and torch."""
     global _calls
     if _calls is None:
         handle = lib()
         with _lock:
             if _calls is None:
-                path = _build.CALLS_PATH
+                path = _build.calls_path()
                 if not os.path.exists(path):
-                    raise ImportError(f"loom-hip call module not found at {path}; run `python -m attnarc_amd.build`")
+                    _calls = _PythonCalls()
+                    return _calls
                 loader = importlib.machinery.ExtensionFileLoader("_loom_hip_calls", path)
                 spec = importlib.util.spec_from_file_location("_loom_hip_calls", path, loader=loader)
                 module = importlib.util.module_from_spec(spec)

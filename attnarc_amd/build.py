@@ -97,7 +97,17 @@ def _compile_adapter(verbose: bool) -> None:
 
 
 CALLS_SOURCE = os.path.join(PKG_DIR, "csrc", "host_calls.cpp")
-CALLS_PATH = os.path.join(PKG_DIR, "_build", "_loom_hip_calls.so")
+
+
+def calls_path() -> str:
+    """The call module's file for this interpreter and torch: it uses both of their C++ ABIs, so its name carries
+    their versions and a build for others is never loaded."""
+    import sys
+
+    import torch
+
+    tag = f"{sys.implementation.cache_tag}-torch{torch.__version__}-cxx11abi{int(torch._C._GLIBCXX_USE_CXX11_ABI)}"
+    return os.path.join(PKG_DIR, "_build", f"_loom_hip_calls.{tag}.so")
 
 
 def _compile_calls(verbose: bool) -> None:
@@ -108,7 +118,8 @@ def _compile_calls(verbose: bool) -> None:
     import torch.utils.cpp_extension as ext
 
     torch_lib = ext.library_paths()[0]
-    tmp = CALLS_PATH + ".tmp"
+    path = calls_path()
+    tmp = path + ".tmp"
     cmd = [
         os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-DUSE_ROCM",
         f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
@@ -122,7 +133,7 @@ def _compile_calls(verbose: bool) -> None:
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True)
-    os.replace(tmp, CALLS_PATH)
+    os.replace(tmp, path)
 
 
 WAVE_TRACE_LIB_PATH = os.path.join(PKG_DIR, "_build", "libloom_hip_wave_trace.so")
