@@ -138,8 +138,9 @@ def paged_decode_attention(
         raise ValueError("paged decode query/value cache must have ranks 3 and 4")
     sequences, query_heads, head_size = query.shape
     value_head_size = value_cache.shape[3]
-    if head_size == value_head_size:
-        output = torch.empty_like(query)  # half the host time of a sized allocation
+    if head_size == value_head_size and type(query) is torch.Tensor:
+        # half the host time of a sized allocation
+        output = torch.empty_like(query, memory_format=torch.contiguous_format)
     else:
         output = torch.empty((sequences, query_heads, value_head_size), device=query.device, dtype=query.dtype)
     _ops._require_inference_tensors(query, key_cache, value_cache)

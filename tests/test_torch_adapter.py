@@ -47,3 +47,22 @@ def test_cpu_tensors_have_no_kernel():
         torch_ops.paged_decode_attention_out(q.requires_grad_(), c, c, torch.zeros(1, 1, dtype=torch.int32),
                                              torch.ones(1, dtype=torch.int32), torch.empty(1, 2, 4),
                                              max_sequence_length=8)
+
+
+def test_decode_output_is_a_plain_contiguous_tensor(monkeypatch):
+    """Whatever strides or subclass the query has (the operator itself needs a GPU: it is left out)."""
+    monkeypatch.setattr(torch_ops, "_paged_decode_attention", lambda *args: None)
+
+    class Tagged(torch.Tensor):
+        pass
+
+    def decode(query):
+        cache = torch.zeros(1, 8, 1, query.shape[2])
+        return torch_ops.paged_decode_attention(query, cache, cache, torch.zeros(1, 1, dtype=torch.int32),
+                                                torch.ones(1, dtype=torch.int32), max_sequence_length=8)
+
+    row = torch.zeros(1, 6, 8)[:, :2]  # one token's query inside a packed row: stride 48 over a size of one
+    for query in (row, torch.zeros(1, 2, 8).as_subclass(Tagged), torch.zeros(2, 3, 8).transpose(0, 1)):
+        out = decode(query)
+        assert type(out) is torch.Tensor and out.shape == query.shape and out.dtype == query.dtype
+        assert out.stride() == (out.shape[1] * 8, 8, 1)
