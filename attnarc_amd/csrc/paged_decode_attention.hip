@@ -54,8 +54,13 @@
 
 #include "../../include/loom_hip.h"
 #include "loom_hip_internal.h"
+#include "stream_plan.h"
 
 namespace {
+
+using loom_hip_decode::StreamCall;
+using loom_hip_decode::StreamPlan;
+using loom_hip_decode::stream_plan;
 
 constexpr float kLog2e = 1.44269504088896340736f;
 constexpr float kLn2 = 0.69314718055994530942f;
@@ -1245,14 +1250,10 @@ constexpr int kStreamStages = 2;
 // One stage per wave (the next step's loads go out when the step has been
 // consumed) holds as many bytes in flight per CU with twice the waves: finer
 // shares, and more waves to compute while others wait. It pays where the items
-// fill the waves. Call us, two stages -> one: head size 256, single waves, 64
-// x 2048 16-bit 180 -> 171, FP8 98.5 -> 91.9, 44 ragged sequences 111 -> 94.8 and
-// 74.8 -> 62.5; head size 128 16-bit (two-item workgroups) 64 x 512-8192 195.8 ->
-// 190.3, 10 x 14000-30000 153.2 -> 149.1, 30 x 32/32 148.7 -> 145.3, but 1,368
-// items 43.6 -> 48.8; FP8 pairs 57 x <= 1998 38.1 -> 33.6, 128 x 4096 188.2 -> 187.9.
-// Head sizes 64-112 keep two (96 NHD ragged 169 -> 175, 64 57 x <= 3000 26.4 ->
-// 39.8).
-constexpr uint64_t kOneStageItems = 2048;
+// fill the waves (stream_plan.h). Call us, two stages -> one: head size 256, single
+// waves, 64 x 2048 16-bit 180 -> 171, FP8 98.5 -> 91.9, 44 ragged sequences 111 ->
+// 94.8 and 74.8 -> 62.5; FP8 pairs 57 x <= 1998 38.1 -> 33.6, 128 x 4096 188.2 ->
+// 187.9.
 
 // kHT: 16-query-head tiles per wave (1, or 2 for groups of 17-32 heads). The
 // tiles share each step's K operand fetches and V transposed reads.
@@ -2509,8 +2510,6 @@ __device__ __forceinline__ void stream_item(const DecodeArgs& a, uint8_t* tiles,
   const uint32_t seq = item.seq;
   const uint32_t len = item.len;
   const uint32_t p0 = part * a.partition_tokens;
-  static_assert(kSplit == 1 || Dec::kWaveBytes >= 16 * (kD + 4) * sizeof(float),
-                "the cross-wave reduction reuses the stages");
 
   Dec dec(a);
   dec.lane = threadIdx.x & 63U;
@@ -2874,7 +2873,10 @@ template <typename QE, bool kFp8, int kSplit, int kHT = 1, uint32_t kD = kDim, i
 __global__ __launch_bounds__(kSplit * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void decode_stream_kernel(DecodeArgs a) {
   using Dec = Decoder<QE, kFp8, kHT, kD, kS, kNt>;
-  __shared__ __attribute__((aligned(16))) uint8_t tiles[kSplit * Dec::kWaveBytes];
+  // The cross-wave reduction reuses the stages (stream_item).
+  constexpr uint32_t kReduceBytes = kSplit > 1 ? 16 * (kD + 4) * sizeof(float) : 0U;
+  __shared__ __attribute__((aligned(16)))
+  uint8_t tiles[kSplit * (Dec::kWaveBytes > kReduceBytes ? Dec::kWaveBytes : kReduceBytes)];
   LOOM_WAVE_STAMP(blockIdx.x * kSplit + (threadIdx.x >> 6));
   const WorkItem item = schedule_item(a, blockIdx.x);
   LOOM_WAVE_ITEM(a, item);
@@ -2895,7 +2897,7 @@ constexpr int kStreamGroup = 4;
 // 94.1 -> 92.4 and 83.4 -> 77.3, 80 106.2 -> 102.3 and 88.2 -> 79.3, 96 106.1 ->
 // 95.4 and 92.7 -> 81.6, 112 95.6 -> 93.3 and 79.0 -> 79.0); two items lose the
 // adjacent heads (96 101.8, 80 122.7). Head size 128 with more than two
-// partitions folds pairs of partitions instead (pair_eligible).
+// partitions folds pairs of partitions instead (folds_pairs).
 
 // kDirect: items in index order (KV head fastest, then partition, then
 // sequence) instead of the longest-first schedule, for the library's own
@@ -3535,38 +3537,19 @@ int launch_mfma_waves(const DecodeArgs& args, uint64_t grid, uint32_t chunks, hi
 // One state per pair halves the split-K state bytes written, which cost far
 // more than their share of the traffic: on C3 the F32 state stores (10.5 MB,
 // 0.9% of the bytes) cost the decode kernel 17 us of 205 (188 us with the
-// stores sent to 32 KiB of L2-resident lines). Measured (C4 call us):
-// eight-item workgroups of four heads x two partitions 201.8 -> 198.4
-// against one state per partition; four-item workgroups of two heads x two
-// partitions then 199.6 -> 194.7 (three pairs; kernel trace 199.1 -> 190.0:
-// three 48 KiB workgroups per CU, where one 96 KiB workgroup per CU ran the
-// launch as four synchronous rounds that dipped at every turnover). 16-bit
-// caches keep one state per partition: two heads x two partitions measured
-// C3 205.5 -> 206.9 us, the loss of four adjacent heads outweighing the
-// halved writes. FP8 at other head sizes neither (call us, pairs against
-// none, B=64, Hq 32 / Hkv 8, 512-token partitions, NHD): head size 64 117.1
-// against 115.3, 80 134.2 against 132.7, 96 131.2 against 129.3, 112 105.5
-// against 104.4.
-bool pair_eligible(const DecodeArgs& a, int group, bool fp8) {
-  // The states are worth folding where a KV head has eight query heads, or four
-  // in an HND cache. Call us, pairs -> none: 16/8 x 1000-2000 x 100 NHD 72.3 ->
-  // 63.6, HND 68.3 -> 62.3, 24/4 NHD 57.6 -> 50.3, 32/32 x <= 1500 NHD 128.6 ->
-  // 125.2, 32/8 NHD 512-8192 111.1 -> 107.9; 32/8 HND 2000-4000 49.3 -> 52.5, 64/8
-  // 33.6 -> 36.7.
-  const bool folds = a.group >= 8 || (a.group >= 4 && a.k_page == a.head_size && a.v_page == a.head_size);
-  return folds && fp8 && a.head_size == kDim && a.parts > 2 && group >= 4 && a.kv_heads % static_cast<uint32_t>(group / 2) == 0;
-}
-
+// stores sent to 32 KiB of L2-resident lines). Which calls fold: folds_pairs.
+// 16-bit caches keep one state per partition: two heads x two
+// partitions measured C3 205.5 -> 206.9 us, the loss of four adjacent heads
+// outweighing the halved writes.
 template <typename QE, bool kFp8, uint32_t kD = kDim, int kGroup = kStreamGroup, int kNt = -1, bool kDirect = false,
           int kS = kStreamStages>
-int launch_stream_group(const DecodeArgs& args, uint64_t items, hipStream_t stream) {
+int launch_stream_group(const DecodeArgs& args, uint64_t items, hipStream_t stream, bool pairs = false) {
   TimedLaunch timed(LOOM_HIP_KERNEL_DECODE, stream);
   g_launch_kernel = "decode_stream_group_kernel";
-  // Pair workgroups exist only as FP8 four-item workgroups at head size 128
-  // (pair_eligible); other instantiations do not compile the pair path.
-  constexpr bool kMayPair = kFp8 && kGroup == 4 && kD == kDim && !kDirect;
-  g_launch_pairs = kMayPair && pair_eligible(args, kGroup, kFp8);
-  if constexpr (kMayPair) {
+  // Pair workgroups exist only as FP8 one-stage workgroups of four items at head
+  // size 128 (folds_pairs); other instantiations do not compile the pair path.
+  if constexpr (kFp8 && kGroup == 4 && kD == kDim && kS == 1) {
+    g_launch_pairs = pairs;
     if (g_launch_pairs) {
       // one workgroup per (sequence, pair of partitions, group of kGroup / 2 KV heads)
       const uint64_t units = (args.parts + 1ULL) / 2ULL * args.sequences * (args.kv_heads / (kGroup / 2));
@@ -3592,42 +3575,62 @@ int launch_stream(const DecodeArgs& args, uint64_t grid, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? LOOM_HIP_SUCCESS : LOOM_HIP_LAUNCH_ERROR;
 }
 
-// Items of fewer than eight 16-token steps on grids that leave CUs idle: four
-// waves share the steps although some take one or none, since a wave alone walks
-// them one after another. Call us, one wave -> four, 100-token contexts: BF16 head
-// size 128 8 items 8.0 -> 6.1, 256 9.0 -> 8.0 (512 9.7 -> 9.9); 64 8 items 6.6 ->
-// 4.9, 512 8.2 -> 7.5; FP8 128 8 items 7.4 -> 5.6, 256 8.5 -> 7.0. 64 tokens: BF16
-// 128 8 items 6.2 -> 5.6, FP8 256 items 6.9 -> 6.8; 33 tokens 6.1 -> 6.4 (BF16, 256
-// items).
-bool short_split(uint64_t grid, uint32_t steps, uint32_t head_size, bool fp8) {
-  return steps < 8 && steps >= (fp8 ? 5U : 4U) && grid <= (head_size == 64 ? 512U : 256U);
-}
-
-// A 4-wave workgroup of head size 80-128 holds 48 KiB or more: from three items
-// per CU one wave per item runs more of them at once (768 and 960 items of 512
-// and 256 tokens, four waves -> one: head size 128 BF16 35.4 -> 30.7 and 28.6 ->
-// 25.3 us, FP8 27.4 -> 23.3 and 23.2 -> 18.9, 96 FP8 27.4 -> 24.4; 512 items BF16
-// 23.6 -> 26.8), for partitions of up to 512 tokens (800 whole sequences of <= 600
-// tokens, 16-bit 96 36.3 -> 37.4).
-bool single_wave(uint64_t grid, uint32_t steps) { return grid >= 768 && steps <= 32; }
-
-// Head sizes 80, 96 and 112 (16-bit cache, one head tile): the launch shapes
-// of head size 128.
+// A plan of stream_plan.h as a launch. kNt: non-temporal hint of the K/V loads
+// (-1: by head size, see StreamDecoder::kNtKV).
 template <typename QE, bool kFp8, uint32_t kD, int kNt = -1>
-int launch_stream_rot_nt(const DecodeArgs& args, uint64_t grid, uint32_t steps, hipStream_t stream) {
-  if (grid >= 4096 || (grid >= 1024 && steps >= 8))
-    return launch_stream_group<QE, kFp8, kD, kStreamGroup, kNt>(args, grid, stream);
-  if ((steps < 8 && !short_split(grid, steps, kD, kFp8)) || single_wave(grid, steps))
-    return launch_stream<QE, kFp8, 1, 1, kD, kNt>(args, grid, stream);
-  return launch_stream<QE, kFp8, 4, 1, kD, kNt>(args, grid, stream);
+int launch_plan_nt(const DecodeArgs& args, const StreamCall& call, const StreamPlan& plan, hipStream_t stream) {
+  const uint64_t n = call.items;
+  if constexpr (kD == 256) {
+    if (plan.items > 1) return launch_stream_group<QE, kFp8, 256, 2, -1, false, 1>(args, n, stream);
+    if (plan.waves > 1) return launch_stream<QE, kFp8, 4, 1, 256>(args, n, stream);
+    return plan.stages == 1 ? launch_stream<QE, kFp8, 1, 1, 256, -1, 1>(args, n, stream)
+                            : launch_stream<QE, kFp8, 1, 1, 256>(args, n, stream);
+  } else {
+    if (plan.items > 1) {
+      if constexpr (kFp8) {
+        return plan.stages == 1
+                   ? launch_stream_group<QE, true, kD, kStreamGroup, kNt, false, 1>(args, n, stream, plan.pairs)
+                   : launch_stream_group<QE, true, kD, kStreamGroup, kNt>(args, n, stream);
+      } else if constexpr (kD == kDim) {
+        // The library's own split runs its items in index order with each
+        // item's first block IDs loaded alongside its length (C2 decode
+        // 18.3-18.5 -> 17.5-17.7 us).
+        if (call.index_order) return launch_stream_group<QE, false, kDim, kStreamGroup, kNt, true>(args, n, stream);
+        if (plan.stages == 1) return launch_stream_group<QE, false, kDim, 2, kNt, false, 1>(args, n, stream);
+      }
+      return launch_stream_group<QE, kFp8, kD, kStreamGroup, kNt>(args, n, stream);
+    }
+    if (plan.waves > 1) {
+      if constexpr (kD > 64) {
+        if (plan.stages == 1) return launch_stream<QE, kFp8, 4, 1, kD, kNt, 1>(args, n, stream);
+      }
+      return launch_stream<QE, kFp8, 4, 1, kD, kNt>(args, n, stream);
+    }
+    return launch_stream<QE, kFp8, 1, 1, kD, kNt, kFp8 ? 1 : kStreamStages>(args, n, stream);
+  }
 }
 
 // Rows that are not whole 128-byte lines take the non-temporal hint only
-// when each KV head's token rows are contiguous (dense_rows: HND).
+// when each KV head's token rows are contiguous (HND: steps cover whole lines).
 template <typename QE, bool kFp8, uint32_t kD>
-int launch_stream_rot(const DecodeArgs& args, uint64_t grid, uint32_t steps, bool dense_rows, hipStream_t stream) {
-  return dense_rows ? launch_stream_rot_nt<QE, kFp8, kD, 1>(args, grid, steps, stream)
-                    : launch_stream_rot_nt<QE, kFp8, kD>(args, grid, steps, stream);
+int launch_plan(const DecodeArgs& args, const StreamCall& call, const StreamPlan& plan, hipStream_t stream) {
+  if constexpr (kD * (kFp8 ? 1U : 2U) % 128U != 0) {
+    if (call.dense) return launch_plan_nt<QE, kFp8, kD, 1>(args, call, plan, stream);
+  }
+  return launch_plan_nt<QE, kFp8, kD>(args, call, plan, stream);
+}
+
+template <typename QE, bool kFp8>
+int launch_streaming(const DecodeArgs& args, const StreamCall& call, hipStream_t stream) {
+  const StreamPlan plan = stream_plan(call);
+  switch (call.head_size) {
+    case 64: return launch_plan<QE, kFp8, 64>(args, call, plan, stream);
+    case 80: return launch_plan<QE, kFp8, 80>(args, call, plan, stream);
+    case 96: return launch_plan<QE, kFp8, 96>(args, call, plan, stream);
+    case 112: return launch_plan<QE, kFp8, 112>(args, call, plan, stream);
+    case 256: return launch_plan<QE, kFp8, 256>(args, call, plan, stream);
+    default: return launch_plan<QE, kFp8, kDim>(args, call, plan, stream);
+  }
 }
 
 // The streaming kernel needs steps that stay inside one block (power-of-two
@@ -3818,7 +3821,7 @@ int launch_f32_stream_nt(const DecodeArgs& args, uint64_t grid, uint32_t steps, 
   constexpr bool kSmall = kD == 64;
   if (grid >= 4096 || (grid >= (kSmall ? 1024 : 2048) && steps >= 8))
     return launch_stream_group<F32Elem, false, kD, kD <= 80 ? 4 : 2, kNt>(args, grid, stream);
-  // Short items share their steps as soon as that saves one (short_split; F32
+  // Short items share their steps as soon as that saves one (splits_short; F32
   // steps are the longest): 33 tokens, one wave -> four, head size 64 8 items 6.5 ->
   // 5.3 us, 512 7.4 -> 7.0; 128 8 items 8.8 -> 7.1, 256 9.0 -> 8.1; two waves at 512
   // items 10.4 -> 9.6.
@@ -3970,102 +3973,26 @@ int run_typed(const Problem& p, hipStream_t stream) {
                      : launch_stream_heads<QE, false, kDim>(args, grid, group, stream);
       }
     }
-  } else if (use_narrow) {
-    if constexpr (!std::is_same<QE, F32Elem>::value) {
-      // Head size 64 or 256, native or FP8 cache: the streaming kernel, in the
-      // launch shapes of the head-size-128 path below.
-      const uint64_t grid = parts * p.kv_heads * static_cast<uint64_t>(p.sequences);
-      if (grid > static_cast<uint64_t>(std::numeric_limits<int>::max()))
-        return fail(LOOM_HIP_UNSUPPORTED, "paged decode grid exceeds the launch limit");
-      args.grid_y = p.kv_heads;
-      const uint32_t steps = (partition_tokens + kStep - 1) / kStep;
-      // Each KV head's token rows contiguous (HND): steps cover whole lines.
-      const bool dense_rows = p.k_page == p.head_size && p.v_page == p.value_head_size;
-      if (p.head_size == 80) {
-        status = fp8 ? launch_stream_rot<QE, true, 80>(args, grid, steps, dense_rows, stream)
-                     : launch_stream_rot<QE, false, 80>(args, grid, steps, dense_rows, stream);
-      } else if (p.head_size == 96) {
-        status = fp8 ? launch_stream_rot<QE, true, 96>(args, grid, steps, dense_rows, stream)
-                     : launch_stream_rot<QE, false, 96>(args, grid, steps, dense_rows, stream);
-      } else if (p.head_size == 112) {
-        status = fp8 ? launch_stream_rot<QE, true, 112>(args, grid, steps, dense_rows, stream)
-                     : launch_stream_rot<QE, false, 112>(args, grid, steps, dense_rows, stream);
-      } else if (p.head_size == 256) {
-        // 16 KiB of LDS per stage: one stage per wave from 1024 items (two
-        // items per workgroup from 4096), and the 4-wave split (two stages,
-        // 129 KiB, one workgroup per CU) for grids under 4 items per CU
-        // (measured: 1024-2048 items ran 11-15% faster as one wave per item;
-        // 128 items 1.6x slower).
-        if (grid >= 4096) {
-          status = fp8 ? launch_stream_group<QE, true, 256, 2, -1, false, 1>(args, grid, stream)
-                       : launch_stream_group<QE, false, 256, 2, -1, false, 1>(args, grid, stream);
-        } else if (grid >= 1024) {
-          status = fp8 ? launch_stream<QE, true, 1, 1, 256, -1, 1>(args, grid, stream)
-                       : launch_stream<QE, false, 1, 1, 256, -1, 1>(args, grid, stream);
-        } else if (steps < 8) {
-          status = fp8 ? launch_stream<QE, true, 1, 1, 256>(args, grid, stream)
-                       : launch_stream<QE, false, 1, 1, 256>(args, grid, stream);
-        } else {
-          status = fp8 ? launch_stream<QE, true, 4, 1, 256>(args, grid, stream)
-                       : launch_stream<QE, false, 4, 1, 256>(args, grid, stream);
-        }
-      } else if (group > 16) {
-        status = fp8 ? launch_stream_heads2<QE, true, 64>(args, grid, stream)
-                     : launch_stream_heads2<QE, false, 64>(args, grid, stream);
-      } else if (grid >= 4096 || (grid >= 1024 && steps >= 8)) {
-        status = fp8 ? (dense_rows ? launch_stream_group<QE, true, 64, kStreamGroup, 1>(args, grid, stream)
-                                   : launch_stream_group<QE, true, 64>(args, grid, stream))
-                     : launch_stream_group<QE, false, 64>(args, grid, stream);
-      } else if (steps < 8 && !short_split(grid, steps, 64, fp8)) {
-        status = fp8 ? (dense_rows ? launch_stream<QE, true, 1, 1, 64, 1>(args, grid, stream)
-                                   : launch_stream<QE, true, 1, 1, 64>(args, grid, stream))
-                     : launch_stream<QE, false, 1, 1, 64>(args, grid, stream);
-      } else {
-        status = fp8 ? (dense_rows ? launch_stream<QE, true, 4, 1, 64, 1>(args, grid, stream)
-                                   : launch_stream<QE, true, 4, 1, 64>(args, grid, stream))
-                     : launch_stream<QE, false, 4, 1, 64>(args, grid, stream);
-      }
-    }
-  } else if (use_mfma) {
+  } else if (use_narrow || use_mfma) {
     if constexpr (!std::is_same<QE, F32Elem>::value) {
     const uint64_t grid = parts * p.kv_heads * static_cast<uint64_t>(p.sequences);
     if (grid > static_cast<uint64_t>(std::numeric_limits<int>::max()))
       return fail(LOOM_HIP_UNSUPPORTED, "paged decode grid exceeds the launch limit");
     args.grid_y = p.kv_heads;
     const uint32_t chunks = (partition_tokens + kChunk - 1) / kChunk;
-    const uint32_t steps = (partition_tokens + kStep - 1) / kStep;
-    if (stream_eligible(p, parts, group)) {
-      // One wave per item, four items (adjacent KV heads) per workgroup, for
-      // grids of 4096 items or more, and from 1024 items (4 per CU) when
-      // partitions have at least 8 steps (measured 10% faster there than the
-      // 4-wave split). Smaller grids split each partition over 4 waves when
-      // that leaves at least 2 steps per wave, else run one wave per
-      // workgroup: there the number of CUs in use matters more than
-      // co-locating heads. (16-wave groups measured slower: they add no CUs,
-      // only contention within one.)
-      if (group > 16) {
+    if (use_narrow || stream_eligible(p, parts, group)) {
+      if (group > 16 && p.head_size == 64) {
+        status = fp8 ? launch_stream_heads2<QE, true, 64>(args, grid, stream)
+                     : launch_stream_heads2<QE, false, 64>(args, grid, stream);
+      } else if (group > 16) {
         status = fp8 ? launch_stream_heads2<QE, true, kDim>(args, grid, stream)
                      : launch_stream_heads2<QE, false, kDim>(args, grid, stream);
-      } else if (grid >= 4096 || (grid >= 1024 && steps >= 8)) {
-        // The library's own split runs its items in index order with each
-        // item's first block IDs loaded alongside its length (C2 decode
-        // 18.3-18.5 -> 17.5-17.7 us).
-        // 16-bit one-stage workgroups of two items: not where partitions are
-        // short or few KV heads lie side by side (20 x <= 14438 in 256-token
-        // partitions 111.5 -> 114.7 us, 300 x 12/2 123.4 -> 130.4, 20 x 20/20
-        // 157.3 -> 163.4) nor under 4,096 items (5 x <= 57468 137.9 -> 143.3).
-        const bool one_stage = fp8 ? grid >= kOneStageItems && steps >= 8
-                                   : grid >= 2 * kOneStageItems && steps >= 32 && p.kv_heads % 8 == 0;
-        status = fp8 ? (one_stage ? launch_stream_group<QE, true, kDim, kStreamGroup, -1, false, 1>(args, grid, stream)
-                                  : launch_stream_group<QE, true>(args, grid, stream))
-                 : one_stage && !p.direct_schedule
-                     ? launch_stream_group<QE, false, kDim, 2, -1, false, 1>(args, grid, stream)
-                 : p.direct_schedule ? launch_stream_group<QE, false, kDim, kStreamGroup, -1, true>(args, grid, stream)
-                                     : launch_stream_group<QE, false>(args, grid, stream);
-      } else if ((steps < 8 && !short_split(grid, steps, kDim, fp8)) || single_wave(grid, steps)) {
-        status = fp8 ? launch_stream<QE, true, 1>(args, grid, stream) : launch_stream<QE, false, 1>(args, grid, stream);
       } else {
-        status = fp8 ? launch_stream<QE, true, 4>(args, grid, stream) : launch_stream<QE, false, 4>(args, grid, stream);
+        const bool dense = p.k_page == p.head_size && p.v_page == p.value_head_size;
+        const StreamCall call{grid, (partition_tokens + kStep - 1) / kStep, p.head_size, group, p.kv_heads, parts, fp8,
+                              dense, p.direct_schedule};
+        status = fp8 ? launch_streaming<QE, true>(args, call, stream)
+                     : launch_streaming<QE, false>(args, call, stream);
       }
     } else if (group > 16) {
       status = fp8 ? launch_mfma_waves<QE, true, 2>(args, grid, chunks, stream)

@@ -1,0 +1,104 @@
+// Launch shape of the streaming decode kernels for groups of up to 16 query heads
+// over 16-bit and FP8 caches, as a function of the call alone. Plain C++, so that a
+// host program can look at any call.
+#pragma once
+
+#include <cstdint>
+
+namespace loom_hip_decode {
+
+struct StreamCall {
+  uint64_t items;        // sequences x partitions x KV heads
+  uint32_t steps;        // 16-token steps of the longest item
+  uint32_t head_size;    // 64, 80, 96, 112, 128 or 256
+  uint32_t group;        // query heads per KV head
+  uint32_t kv_heads;
+  uint64_t parts;        // partitions of the longest sequence
+  bool fp8;              // FP8 cache, else 16-bit
+  bool dense;            // each KV head's token rows are contiguous (HND)
+  bool index_order;      // the library's own split: items in index order
+};
+
+struct StreamPlan {
+  uint32_t waves;   // per item
+  uint32_t items;   // per workgroup (one wave each where more than one)
+  uint32_t stages;  // pipeline stages per wave
+  bool pairs;       // a workgroup folds two consecutive partitions of two KV heads
+};
+
+// What decides is how many items a CU holds at once. A stage takes 8 KiB of LDS at
+// head size 128 (16 tokens of a 16-bit cache, 32 of an FP8 one), so a CU holds two
+// workgroups of four two-stage waves, and four of one-stage waves; two stages hide
+// more of a load's latency. Sequence lengths are on the device: a ragged batch has
+// fewer and shorter items than the call says. Figures below are geometric means of
+// call times over some 30,000 calls of generic shapes; those of FP8 caches are
+// relative to the form with steps of 16 tokens (see Fp8StreamDecoder), whose
+// two-stage waves took 12 KiB.
+
+// FP8 workgroups fold pairs of partitions (pair_item, head size 128) where the
+// states they save are worth the coarser workgroups: all short partitions, and
+// groups of more than four heads, or four in an HND cache, where a partition
+// holds eight steps or more. None -> pairs (one stage): four-step partitions, 1 head
+// 0.83 -> 0.83, 2 0.85 -> 0.85, 6 0.97 -> 0.86, 8 1.04 -> 0.87; eight steps from 4,096
+// items, NHD, 1 / 2 / 4 heads 0.88 / 0.90 / 0.94 -> 0.89 / 0.88 / 0.93, 6 1.01 -> 0.92, 8
+// 0.98 -> 0.92; HND, 4 0.94 -> 0.89, 6 0.97 -> 0.90.
+inline bool folds_pairs(const StreamCall& c) {
+  if (!c.fp8 || c.head_size != 128 || c.parts <= 2 || c.kv_heads % 2 != 0) return false;
+  return c.steps < 8 || c.group > 4 || (c.group == 4 && c.dense);
+}
+
+// Items of fewer than eight steps on grids that leave CUs idle: four waves share
+// the steps although some take one or none, since a wave alone walks them one
+// after another. Call us, one wave -> four, 100-token contexts: BF16 head size 128 8
+// items 8.0 -> 6.1, 256 9.0 -> 8.0 (512 9.7 -> 9.9); 64 8 items 6.6 -> 4.9, 512 8.2 ->
+// 7.5; FP8 128 8 items 7.4 -> 5.6, 256 8.5 -> 7.0.
+inline bool splits_short(const StreamCall& c) {
+  if (c.steps >= 8 || c.items > (c.head_size == 64 ? 512U : 256U)) return false;
+  return c.steps >= (c.fp8 ? 5U : 4U);
+}
+
+inline StreamPlan stream_plan(const StreamCall& c) {
+  const bool grouped = c.items >= 4096 || (c.items >= 1024 && c.steps >= 8);
+  if (c.head_size == 256) {
+    // A stage takes 16 KiB: five two-stage waves fit a CU, ten one-stage ones.
+    // The 4-wave split under 4 items per CU (128 items as single waves 1.6x slower).
+    if (c.items >= 4096) return {1, 2, 1, false};
+    if (c.items >= 1024) return {1, 1, 1, false};
+    return c.steps < 8 ? StreamPlan{1, 1, 2, false} : StreamPlan{4, 1, 2, false};
+  }
+  if (grouped && c.fp8) {
+    // One stage where items are short or fill the waves. Two stages -> one: four
+    // steps at 128 1.06 -> 0.85 (as pairs), 64 1.00 -> 0.90, 112 0.85 -> 0.64; from
+    // 4,096 items, 8 / 16 steps, 64 0.98 / 0.94 -> 0.91 / 0.90, 96 0.71 / 0.68 -> 0.65 / 0.63,
+    // 128 0.98 / 0.93 -> 0.89 / 0.88; 2,048-4,095 at 64 0.83 -> 0.86, at 128 0.88 -> 0.82;
+    // pairs of 1,024-2,047 items 0.87 -> 0.87, the worst call 1.10 -> 0.93.
+    const bool pairs = folds_pairs(c);
+    const bool one = pairs || c.steps < 8 || c.items >= (c.head_size == 128 ? 2048U : 4096U);
+    return {1, 4, one ? 1U : 2U, pairs};
+  }
+  if (grouped) {
+    // 16-bit one-stage waves, two items to a workgroup.
+    const bool one = c.head_size == 128 && !c.index_order && c.items >= 4096 && c.steps >= 32 && c.kv_heads % 8 == 0;
+    return one ? StreamPlan{1, 2, 1, false} : StreamPlan{1, 4, 2, false};
+  }
+  if (c.steps < 8 && !splits_short(c)) {
+    // FP8: one 32-token step, or a few, in half the LDS. Two stages -> one at 128:
+    // 2,560-4,095 items of 1 / 2 / 4 steps 1.22 / 1.16 / 0.99 -> 0.91 / 0.86 / 0.88,
+    // 257-512 items 1.02 / 0.94 / 0.90 -> 0.98 / 0.91 / 0.87.
+    return {1, 1, c.fp8 ? 1U : 2U, false};
+  }
+  if (c.fp8) {
+    // Past two 64 KiB workgroups per CU. Two stages -> one at 80-128, 513-767 items
+    // of 16 / 32 / 64 steps 1.02 / 0.98 / 0.91 -> 0.90 / 0.89 / 0.88, 768-1,023 1.00 / 0.93 /
+    // 0.91 -> 0.81 / 0.82 / 0.85 (as single waves 0.80 / 0.88 / 0.95, ragged batches up to
+    // 1.43); at 64 (32 KiB) 0.93 and 0.93.
+    return {4, 1, c.head_size > 64 && c.items > 512 ? 1U : 2U, false};
+  }
+  // 16-bit caches, from three items per CU: one wave per item runs more of them at
+  // once (768 and 960 items of 512 and 256 tokens at 128 35.4 -> 30.7 and 28.6 ->
+  // 25.3 us; 512 items 23.6 -> 26.8), for partitions of up to 512 tokens.
+  const bool single = c.items >= 768 && c.steps <= 32 && c.head_size > 64;
+  return single ? StreamPlan{1, 1, 2, false} : StreamPlan{4, 1, 2, false};
+}
+
+}  // namespace loom_hip_decode

@@ -126,9 +126,10 @@ def test_length_past_max_sequence_length_stays_in_its_share(hq, hkv, dtype):
 @pytest.mark.parametrize("head,layout,hkv", [(128, "HND", 8), (128, "NHD", 8), (64, "HND", 8), (128, "HND", 6),
                                              (128, "NHD", 3)])
 def test_fp8_two_partition_workgroups(head, layout, hkv):
-    """FP8 grids of 1024+ items at head size 128 run four-item workgroups of
-    two KV heads x two partitions that leave one state per pair (head size
-    64: eight-item workgroups, one state per partition): sequences that end
+    """FP8 grids of 1024+ items at head size 128 run four-item workgroups, in HND
+    order with an even number of KV heads as two KV heads x two partitions that
+    leave one state per pair (else, and at head size 64, one state per
+    partition): sequences that end
     inside the first partition of a pair, exactly on a pair boundary, one
     token past it, and single-token ones."""
     rng = np.random.default_rng(head)
