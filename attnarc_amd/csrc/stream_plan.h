@@ -61,9 +61,11 @@ inline StreamPlan stream_plan(const StreamCall& c) {
   const bool grouped = c.items >= 4096 || (c.items >= 1024 && c.steps >= 8);
   if (c.head_size == 256) {
     // A stage takes 16 KiB: five two-stage waves fit a CU, ten one-stage ones.
-    // The 4-wave split under 4 items per CU (128 items as single waves 1.6x slower).
+    // 1,025-1,280 items, two stages -> one: ragged 16-bit 0.98 -> 1.07, fixed
+    // lengths 0.99 -> 0.89; FP8 0.95 -> 0.88. The 4-wave split under 4 items per
+    // CU (128 items as single waves 1.6x slower).
     if (c.items >= 4096) return {1, 2, 1, false};
-    if (c.items >= 1024) return {1, 1, 1, false};
+    if (c.items >= 1024) return {1, 1, c.fp8 || c.items > 1280 ? 1U : 2U, false};
     return c.steps < 8 ? StreamPlan{1, 1, 2, false} : StreamPlan{4, 1, 2, false};
   }
   if (grouped && c.fp8) {
@@ -94,11 +96,13 @@ inline StreamPlan stream_plan(const StreamCall& c) {
     // 1.43); at 64 (32 KiB) 0.93 and 0.93.
     return {4, 1, c.head_size > 64 && c.items > 512 ? 1U : 2U, false};
   }
-  // 16-bit caches, from three items per CU: one wave per item runs more of them at
-  // once (768 and 960 items of 512 and 256 tokens at 128 35.4 -> 30.7 and 28.6 ->
-  // 25.3 us; 512 items 23.6 -> 26.8), for partitions of up to 512 tokens.
-  const bool single = c.items >= 768 && c.steps <= 32 && c.head_size > 64;
-  return single ? StreamPlan{1, 1, 2, false} : StreamPlan{4, 1, 2, false};
+  // 16-bit caches, from three items per CU: more of them at once on one-stage
+  // waves. Two stages -> one at 128, 8 / 16 / 32 steps: fixed lengths 0.81 / 0.89 /
+  // 0.95, ragged 0.83 / 0.82 / 0.97; at 80 (48 KiB, three per CU) 0.84 / 0.93 / 0.97 and
+  // 1.00 / 0.93 / 1.02. (Single waves at 128: fixed 0.75 / 0.85 / 0.93, but ragged
+  // batches up to 1.30, at 80 up to 1.43.)
+  const bool one = c.items >= 768 && c.steps <= (c.head_size >= 112 ? 32U : 24U) && c.head_size > 64;
+  return {4, 1, one ? 1U : 2U, false};
 }
 
 }  // namespace loom_hip_decode

@@ -20,12 +20,16 @@ SHAPES = [
     (("fp8", 130, (24, 4), 128, 384, 128, "NHD"), PAIRS),
     (("fp8", 130, (16, 4), 128, 384, 128, "HND"), PAIRS),
     (("fp8", 130, (16, 4), 128, 384, 128, "NHD"), GROUP_TWO),
+    *[(("native", 96, (16, 8), d, 300, 0, "HND" if d == 80 else "NHD"), SPLIT) for d in (80, 96, 112, 128)],
     (("native", 96, (16, 8), 64, 300, 0, "NHD"), SPLIT_TWO),
     (("native", 191, (8, 4), 128, 300, 0, "NHD"), SPLIT_TWO),
+    (("native", 96, (16, 8), 96, 400, 0, "NHD"), SPLIT_TWO),
+    (("native", 96, (16, 8), 112, 400, 0, "NHD"), SPLIT),
     (("native", 20, (16, 1), 128, 112, 0, "NHD"), SPLIT_TWO),
     (("native", 20, (8, 1), 96, 80, 0, "HND"), SPLIT_TWO),
     (("native", 20, (12, 2), 128, 64, 0, "NHD"), SPLIT_TWO),
     (("native", 171, (64, 16), 128, 1030, 512, "NHD"), GROUP_OF_TWO),
+    (("native", 320, (8, 4), 256, 200, 0, "NHD"), SINGLE_TWO),
     (("native", 321, (8, 4), 256, 200, 0, "NHD"), SINGLE),
     (("fp8", 256, (8, 4), 256, 200, 0, "NHD"), SINGLE),
 ]

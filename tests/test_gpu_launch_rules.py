@@ -1,7 +1,8 @@
 """Shapes on both sides of the streaming kernels' launch rules, against the CPU oracle.
 
-Short items shared by four waves (two for large F32 rows), single waves from
-768 items, and FP8 pairs of partitions by group size and cache layout.
+Short items shared by four waves (two for large F32 rows), four waves on one or
+two stages either side of 768 items, and FP8 pairs of partitions by group size and
+cache layout.
 """
 
 from __future__ import annotations

@@ -50,6 +50,9 @@ def test_library_split_keeps_index_order(plan_of):
     (("fp8", 22, (32, 32), 128, 160, 0, "NHD"), SPLIT),        # 12.9 on two stages, 9.0
     (("fp8", 21, (20, 20), 128, 525, 512, "NHD"), SPLIT),      # 21.7 on single waves, 15.5
     (("fp8", 80, (64, 8), 112, 149, 0, "NHD"), SPLIT),         # 15.7 on two stages, 10.5
+    (("native", 13, (20, 20), 96, 1310, 512, "HND"), SPLIT_TWO),  # 23.7 on single waves, 17.5
+    (("native", 19, (16, 8), 80, 1325, 256, "HND"), SPLIT),    # 14.9 on single waves, 11.5
+    (("native", 17, (32, 32), 256, 617, 512, "NHD"), SINGLE_TWO),  # 52.5 on one stage, 40.0
 ])
 def test_shapes_that_were_slower(plan_of, shape, want):
     assert plan_of(*shape) == want
