@@ -49,12 +49,17 @@ inline bool folds_pairs(const StreamCall& c) {
 
 // Items of fewer than eight steps on grids that leave CUs idle: four waves share
 // the steps although some take one or none, since a wave alone walks them one
-// after another. Call us, one wave -> four, 100-token contexts: BF16 head size 128 8
+// after another. The reduction costs more with more heads, so wide groups need
+// more steps. Call us, one wave -> four, 100-token contexts: BF16 head size 128 8
 // items 8.0 -> 6.1, 256 9.0 -> 8.0 (512 9.7 -> 9.9); 64 8 items 6.6 -> 4.9, 512 8.2 ->
-// 7.5; FP8 128 8 items 7.4 -> 5.6, 256 8.5 -> 7.0.
+// 7.5; FP8 128 8 items 7.4 -> 5.6, 256 8.5 -> 7.0. Four waves over one by group and
+// steps, up to 256 items: 16-bit 2 heads 0.91 / 0.83 at 4 / 5 steps, 8 heads 1.01 /
+// 0.94, 16 heads 1.13 / 1.06 / 1.03 / 0.91 at 4 / 5 / 6 / 7; FP8 8 heads 0.82 at 5, 16
+// heads 0.96 / 0.85 at 5 / 6.
 inline bool splits_short(const StreamCall& c) {
   if (c.steps >= 8 || c.items > (c.head_size == 64 ? 512U : 256U)) return false;
-  return c.steps >= (c.fp8 ? 5U : 4U);
+  if (c.fp8) return c.steps >= (c.group > 8 ? 6U : 5U);
+  return c.steps >= (c.group > 8 ? 7U : c.group > 6 ? 5U : 4U);
 }
 
 inline StreamPlan stream_plan(const StreamCall& c) {

@@ -12,6 +12,7 @@ SHAPES = [
     (("fp8", 128, (8, 4), 128, 300, 0, "NHD"), SPLIT_TWO),
     (("fp8", 65, (8, 4), 128, 112, 0, "NHD"), SINGLE),
     *[(("fp8", 129, (8, 4), d, 97, 0, "NHD" if d == 80 else "HND"), SINGLE) for d in (64, 80, 96, 112, 128)],
+    (("fp8", 20, (16, 1), 128, 80, 0, "NHD"), SINGLE),
     (("fp8", 20, (16, 1), 128, 96, 0, "NHD"), SPLIT_TWO),
     *[(("fp8", 260, (16, 8), d, 128, 64, "HND" if d == 112 else "NHD"), GROUP) for d in (64, 80, 96, 112, 128)],
     (("fp8", 520, (8, 8), 96, 300, 0, "NHD"), GROUP),
@@ -25,7 +26,9 @@ SHAPES = [
     (("native", 191, (8, 4), 128, 300, 0, "NHD"), SPLIT_TWO),
     (("native", 96, (16, 8), 96, 400, 0, "NHD"), SPLIT_TWO),
     (("native", 96, (16, 8), 112, 400, 0, "NHD"), SPLIT),
+    (("native", 20, (16, 1), 128, 96, 0, "NHD"), SINGLE_TWO),
     (("native", 20, (16, 1), 128, 112, 0, "NHD"), SPLIT_TWO),
+    (("native", 20, (8, 1), 96, 64, 0, "HND"), SINGLE_TWO),
     (("native", 20, (8, 1), 96, 80, 0, "HND"), SPLIT_TWO),
     (("native", 20, (12, 2), 128, 64, 0, "NHD"), SPLIT_TWO),
     (("native", 171, (64, 16), 128, 1030, 512, "NHD"), GROUP_OF_TWO),
