@@ -84,8 +84,11 @@ inline StreamPlan stream_plan(const StreamCall& c) {
     return {1, 4, one ? 1U : 2U, pairs};
   }
   if (grouped) {
-    // 16-bit one-stage waves, two items to a workgroup.
-    const bool one = c.head_size == 128 && !c.index_order && c.items >= 4096 && c.steps >= 32 && c.kv_heads % 8 == 0;
+    // 16-bit one-stage waves, two items to a workgroup, over two-stage ones, four to
+    // a workgroup: from 8,192 items (four rounds of the latter) 0.98, at most 1.01,
+    // for groups of four heads and more; 1.02 and up to 1.09 for fewer, and between
+    // 4,096 and 8,191 0.96-1.05 by how the last round fills, up to 1.11.
+    const bool one = c.head_size == 128 && !c.index_order && c.items >= 8192 && c.steps >= 32 && c.group >= 4;
     return one ? StreamPlan{1, 2, 1, false} : StreamPlan{1, 4, 2, false};
   }
   if (c.steps < 8 && !splits_short(c)) {

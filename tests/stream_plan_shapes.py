@@ -32,6 +32,7 @@ SHAPES = [
     (("native", 20, (8, 1), 96, 80, 0, "HND"), SPLIT_TWO),
     (("native", 20, (12, 2), 128, 64, 0, "NHD"), SPLIT_TWO),
     (("native", 171, (64, 16), 128, 1030, 512, "NHD"), GROUP_OF_TWO),
+    (("native", 170, (64, 16), 128, 1030, 512, "HND"), GROUP_TWO),
     (("native", 320, (8, 4), 256, 200, 0, "NHD"), SINGLE_TWO),
     (("native", 321, (8, 4), 256, 200, 0, "NHD"), SINGLE),
     (("fp8", 256, (8, 4), 256, 200, 0, "NHD"), SINGLE),

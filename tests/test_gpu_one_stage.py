@@ -1,9 +1,11 @@
 """Streaming waves with one pipeline stage, on grids large enough to take them.
 
-At head size 128 from 2,048 items (FP8; 4,096 of 512 tokens or more for 16-bit
-caches with a multiple of eight KV heads) and at 256 from 1,024 a wave refills
-its only stage after each step. Ragged lengths end items in every step remainder. Against
-the CPU oracle at the bars of the other parity tests.
+At head size 128 FP8 items from 2,048 (1,024 as pairs of partitions) and at 256
+FP8 items from 1,024 and 16-bit ones from 1,281 run on waves that refill their only
+stage after each step. (The 16-bit rows at 128 are too short for it: they run two
+stages. test_gpu_stream_plans.py has the shapes of every launch.) Ragged lengths end
+items in every step remainder. Against the CPU oracle at the bars of the other
+parity tests.
 """
 
 from __future__ import annotations
@@ -25,7 +27,7 @@ DEV = "cuda:0"
     (255, (6, 3), 128, 128, "decode_stream_group_kernel"),  # 2,295 items, an odd head count
     (260, (16, 8), 128, 0, "decode_stream_group_kernel"),   # 2,080 whole sequences
     (516, (8, 8), 128, 512, "decode_stream_group_kernel"),  # 4,128 whole sequences
-    (171, (16, 8), 128, 512, "decode_stream_group_kernel"),  # 1,368 items: two stages
+    (171, (16, 8), 128, 512, "decode_stream_group_kernel"),  # 1,368 whole sequences: two stages
     (259, (4, 2), 256, 128, "decode_stream_kernel"),        # 1,554 items
     (512, (8, 4), 256, 128, "decode_stream_group_kernel"),  # 6,144 items
 ])

@@ -54,6 +54,8 @@ def test_library_split_keeps_index_order(plan_of):
     (("native", 19, (16, 8), 80, 1325, 256, "HND"), SPLIT),    # 14.9 on single waves, 11.5
     (("native", 17, (32, 32), 256, 617, 512, "NHD"), SINGLE_TWO),  # 52.5 on one stage, 40.0
     (("native", 18, (16, 1), 128, 387, 64, "NHD"), SINGLE_TWO),  # 10.9 on four waves, 8.7
+    (("native", 340, (16, 8), 128, 1000, 512, "NHD"), GROUP_TWO),  # one-stage waves up to 1.1 times as long
+    (("native", 1100, (8, 8), 128, 520, 0, "HND"), GROUP_TWO),
 ])
 def test_shapes_that_were_slower(plan_of, shape, want):
     assert plan_of(*shape) == want
