@@ -77,10 +77,13 @@ inline StreamPlan stream_plan(const StreamCall& c) {
     // One stage where items are short or fill the waves. Two stages -> one: four
     // steps at 128 1.06 -> 0.85 (as pairs), 64 1.00 -> 0.90, 112 0.85 -> 0.64; from
     // 4,096 items, 8 / 16 steps, 64 0.98 / 0.94 -> 0.91 / 0.90, 96 0.71 / 0.68 -> 0.65 / 0.63,
-    // 128 0.98 / 0.93 -> 0.89 / 0.88; 2,048-4,095 at 64 0.83 -> 0.86, at 128 0.88 -> 0.82;
+    // 128 0.98 / 0.93 -> 0.89 / 0.88; but 32 steps at 80 and 96 0.70 / 0.76 -> 0.71 / 0.77
+    // (32 x <= 4,001 tokens of 32/32 heads at 96 100.6 -> 102.9 us); 2,048-4,095 items at
+    // 64 0.83 -> 0.86, at 128 0.88 -> 0.82;
     // pairs of 1,024-2,047 items 0.87 -> 0.87, the worst call 1.10 -> 0.93.
     const bool pairs = folds_pairs(c);
-    const bool one = pairs || c.steps < 8 || c.items >= (c.head_size == 128 ? 2048U : 4096U);
+    const bool one = pairs || c.steps < 8 ||
+                     (c.head_size == 128 ? c.items >= 2048 : c.items >= 4096 && c.steps <= 16);
     return {1, 4, one ? 1U : 2U, pairs};
   }
   if (grouped) {

@@ -15,7 +15,8 @@ SHAPES = [
     (("fp8", 20, (16, 1), 128, 80, 0, "NHD"), SINGLE),
     (("fp8", 20, (16, 1), 128, 96, 0, "NHD"), SPLIT_TWO),
     *[(("fp8", 260, (16, 8), d, 128, 64, "HND" if d == 112 else "NHD"), GROUP) for d in (64, 80, 96, 112, 128)],
-    (("fp8", 520, (8, 8), 96, 300, 0, "NHD"), GROUP),
+    (("fp8", 520, (8, 8), 96, 256, 0, "NHD"), GROUP),
+    (("fp8", 520, (8, 8), 96, 257, 0, "NHD"), GROUP_TWO),
     (("fp8", 260, (8, 8), 96, 300, 0, "NHD"), GROUP_TWO),
     (("fp8", 180, (8, 8), 128, 150, 64, "NHD"), PAIRS),
     (("fp8", 130, (24, 4), 128, 384, 128, "NHD"), PAIRS),
