@@ -1639,9 +1639,10 @@ struct F32StreamDecoder {
   static constexpr uint32_t kWaveBytes = kStages * kStageBytes;
   static constexpr int kDmaPerStep = 2 * kDma;
   static constexpr uint32_t kElem = 4;
-  // K row r keeps chunk L at (L + (r >> kRotShift)) mod kRowChunks: the 16
-  // rows of one operand read then cover all banks (row pitches repeat over the
-  // 256 bytes of banks after 1, 2 or 4 rows). V rows are read along the row.
+  // K row r keeps chunk L at (L + (r >> kRotShift)) mod kRowChunks, which spreads
+  // the 16 rows of one operand read over the banks (row pitches repeat over the 256
+  // bytes of banks after 1, 2 or 4 rows). V rows are read along the row. At 128 a step
+  // reads 32 conflict cycles of 97 active.
   static constexpr uint32_t kRotShift = kPitch % 256U == 0 ? 0U : kPitch % 128U == 0 ? 1U : 2U;
 
   const DecodeArgs& a;
@@ -1858,8 +1859,9 @@ struct Fp8StreamDecoder {
   static constexpr uint32_t kTailLanes = kHalfBytes % 1024 == 0 ? 64U : kHalfBytes % 1024 / 16;
   static constexpr int kDmaPerHalf = 2 * kDma;
   // A stage: K of both halves, then V of both. Unswizzled V rows (80-112
-  // bytes) put half 1 where its eight rows of a transposed read fall on the
-  // 16-byte bank slots that half 0's leave free.
+  // bytes) put half 1 where its eight rows of a transposed read fall on other
+  // 16-byte bank slots than half 0's. (At 96 a step still reads 72 conflict cycles
+  // of 110 active, K's 96-byte rows among them.)
   static constexpr uint32_t kVOff = 2 * kHalfBytes;
   static constexpr uint32_t kVOff1 = 3 * kHalfBytes + (kSwz ? 0U : kD == 96 ? 16U : 128U);
   static constexpr int kStages = kS;
@@ -1908,8 +1910,10 @@ struct Fp8StreamDecoder {
   }
 
   // Chunk L of row r sits at L ^ k_swizzle(r) in K, L ^ v_swizzle(b, r) in V
-  // of half b: the 8-byte K operand reads of 16 rows, and the transposed reads
-  // of eight rows of both halves, then cover distinct banks.
+  // of half b, which spreads the 8-byte K operand reads of 16 rows and the
+  // transposed reads of eight rows of both halves over the banks. Counters still
+  // read four conflict cycles per 16 dims of a step (at 128 32 of its 85 LDS
+  // cycles); the LDS does not bound these kernels.
   static __device__ __forceinline__ uint32_t k_swizzle(uint32_t r) {
     return kD == 256 ? (r & 15U) : kD == 128 ? ((r >> 1) & 7U) : kD == 64 ? ((r >> 2) & 3U) : 0U;
   }
